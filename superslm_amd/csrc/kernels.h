@@ -69,7 +69,7 @@ struct GemmArgs {
 	const int8_t* a;   // [M, K] activation codes, row stride lda
 	const int8_t* w;   // [N, K] weights
 	// the same weights in the packed decode layout (k_gemv_pk in kernels.hip), or null; decode
-	// GEMVs at M <= 32 read them instead of w
+	// GEMVs at M <= 128 read them instead of w
 	const int8_t* wp;
 	int32_t M, N, K, lda;
 	Epilogue epi;
@@ -140,8 +140,12 @@ void gemm(const GemmArgs& g, hipStream_t s);
 // argmax keys)
 GemvPlan gemv_plan(int M, int N, int K, bool split_ok, bool raw_or_argmax = false);
 bool gemv_eligible(int M, int K);
+// Planes the packed decode kernels write for a raw launch of M tokens on an [N, K] matrix with a
+// packed copy (1 = a single plane); 0 when they do not take the shape.
+int packed_planes(int M, int N, int K);
 // Split-K planes a raw decode GEMV writes for a consumer that adds them: the packed kernels' plan
-// when g.wp is set and they take the launch, else gemv_plan's.  1 = a single plane.
+// when g.wp is set and they take the launch, else gemv_plan's.  1 = a single plane, 0 = no decode
+// GEMV takes the launch.
 int gemv_raw_splits(const GemmArgs& g);
 // bytes of the packed decode copy of an [N, K] matrix (whole 16-row tiles)
 size_t packed_bytes(int N, int K);
@@ -340,7 +344,7 @@ struct ActArgs {
 	SiteTap gate_tap, up_tap;  // the gate / up funnels' codes and scales
 };
 constexpr int kMaxActSlices = 16;
-constexpr int kMaxSlicedActRows = 64;  // rows the sliced form's buffers hold
+constexpr int kMaxSlicedActRows = 128;  // rows the sliced form's buffers hold
 void mlp_act(const ActArgs& a, hipStream_t s);
 // The same step on every row cut into column slices, one block per (row, slice), in two
 // launches: gate and up funnels, SiLU products and per-slice maxima; then the act funnel over the

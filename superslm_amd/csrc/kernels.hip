@@ -541,7 +541,7 @@ __global__ __launch_bounds__(256) void k_gemv_p(GemmArgs g) {
 }
 
 // ------------------------------------------------------------------------------------------
-// LM head on the packed decode copy (M <= 32, K <= 4096), persistent: one block per CU walks the
+// LM head on the packed decode copy (M <= 128, K <= 4096), persistent: one block per CU walks the
 // 16-column tiles blockIdx.x, + gridDim.x, ...; wave w keeps K chunks w CPW .. + CPW of the MB
 // 16-token row groups in registers for the whole launch and loads the next tile's weight chunks
 // while it multiplies the current tile's, two register sets alternating (the loop body is two
@@ -555,31 +555,39 @@ __device__ __forceinline__ const int8_t* pk_lane(const int8_t* wp, int tile, int
 
 constexpr int kHeadMaxSteps = 64;  // tiles per block of k_gemv_head (the launch sizes its grid to fit)
 
-template <int MB, int CPW>
-__global__ __launch_bounds__(256) void k_gemv_head(GemmArgs g) {
-	__shared__ v4i red[2][kGemvWaves][MB][64];
+// Four row groups (M 33..64) over more than 16 chunks take eight waves of CPW chunks (NW = 8, as in
+// k_gemv_pk), wave w finishing token row w % 4 of row groups w / 4, w / 4 + 2.
+template <int MB, int CPW, int NW = kGemvWaves>
+__global__ __launch_bounds__(64 * NW) void k_gemv_head(GemmArgs g) {
+	static_assert(NW == kGemvWaves || (NW == 2 * kGemvWaves && MB % 2 == 0), "eight waves share the row groups evenly");
+	constexpr int MW = MB * kGemvWaves / NW;  // row groups this wave finishes: mb_of(0), ...
+	__shared__ v4i red[2][NW][MB][64];
 	// the block's keys, stored after the loop: a global store inside it (stores count in the
 	// vector-memory counter) left the waits before each step's MFMAs draining the next tile's loads
 	__shared__ uint64_t s_key[kHeadMaxSteps][MB * 16];
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ri = lane & 15, grp = lane >> 4;
 	const int C = g.K >> 7, T = (g.N + 15) / 16;
 	const v4i z = v4i{0, 0, 0, 0};
+	// this block's first token, and the tokens from it (row blocks: launches past 64 tokens)
+	const int m0 = MB == 4 ? blockIdx.y * (MB * 16) : 0, M = g.M - m0;
 	const Epilogue& e = g.epi;
 	// this lane's epilogue tokens (mb * 16 + 4 grp + wave) and their schema pages: a mask byte
 	// travels with each tile's weights, read from a valid address whether or not a page is set, so
 	// no wait inside the loop drains the next tile's loads
-	const uint8_t* pgp[MB];
-	bool masked[MB];
+	const int row4 = wave & 3;
+	auto mb_of = [&](int u) { return NW == kGemvWaves ? u : (wave >> 2) + 2 * u; };
+	const uint8_t* pgp[MW];
+	bool masked[MW];
 #pragma unroll
-	for (int mb = 0; mb < MB; ++mb) {
-		const int tk = min(mb * 16 + grp * 4 + wave, g.M - 1);
+	for (int u = 0; u < MW; ++u) {
+		const int tk = m0 + min(mb_of(u) * 16 + grp * 4 + row4, M - 1);
 		const uint8_t* pg = e.mask_page ? e.mask_page[tk] : nullptr;
-		masked[mb] = pg != nullptr;
-		pgp[mb] = pg ? pg : (const uint8_t*)g.wp;
+		masked[u] = pg != nullptr;
+		pgp[u] = pg ? pg : (const uint8_t*)g.wp;
 	}
 	struct Tile {
 		v4i b[CPW][2];
-		uint8_t mbits[MB];
+		uint8_t mbits[MW];
 	};
 	auto load_tile = [&](int t, Tile& d) {
 		const int tc = min(t, T - 1);
@@ -594,8 +602,8 @@ __global__ __launch_bounds__(256) void k_gemv_head(GemmArgs g) {
 		// a global-space load: through a generic pointer it would be a flat load, which counts in
 		// both wait counters and made every LDS wait of the epilogue drain the weight loads
 #pragma unroll
-		for (int mb = 0; mb < MB; ++mb)
-			d.mbits[mb] = ((const __attribute__((address_space(1))) uint8_t*)pgp[mb])[masked[mb] ? jm : 0];
+		for (int u = 0; u < MW; ++u)
+			d.mbits[u] = ((const __attribute__((address_space(1))) uint8_t*)pgp[u])[masked[u] ? jm : 0];
 	};
 	Tile t0buf, t1buf;
 	int tile = blockIdx.x, it = 0;
@@ -604,8 +612,8 @@ __global__ __launch_bounds__(256) void k_gemv_head(GemmArgs g) {
 #pragma unroll
 	for (int mb = 0; mb < MB; ++mb) {
 		const int r = mb * 16 + ri;
-		const bool rok = r < g.M;
-		const int8_t* arow = g.a + (size_t)(rok ? r : g.M - 1) * g.lda + grp * 16;
+		const bool rok = r < M;
+		const int8_t* arow = g.a + (size_t)(m0 + (rok ? r : M - 1)) * g.lda + grp * 16;
 #pragma unroll
 		for (int i = 0; i < CPW; ++i) {
 			const int c = wave * CPW + i;
@@ -631,12 +639,13 @@ __global__ __launch_bounds__(256) void k_gemv_head(GemmArgs g) {
 		__syncthreads();
 		const int j = tl * 16 + ri;
 #pragma unroll
-		for (int mb = 0; mb < MB; ++mb) {
+		for (int u = 0; u < MW; ++u) {
+			const int mb = mb_of(u);
 			int32_t tot = 0;
 #pragma unroll
-			for (int w = 0; w < kGemvWaves; ++w) tot += ((const int32_t*)&red[k & 1][w][mb][lane])[wave];
-			const int tk = mb * 16 + grp * 4 + wave;
-			const int32_t lv = masked[mb] && j < g.N && !((cur.mbits[mb] >> (j & 7)) & 1u) ? INT32_MIN : tot;
+			for (int w = 0; w < NW; ++w) tot += ((const int32_t*)&red[k & 1][w][mb][lane])[row4];
+			const int tk = mb * 16 + grp * 4 + row4;
+			const int32_t lv = masked[u] && j < g.N && !((cur.mbits[u] >> (j & 7)) & 1u) ? INT32_MIN : tot;
 			uint64_t key = j < g.N ? ((uint64_t)((uint32_t)lv ^ 0x80000000u) << 32) | (0xffffffffu - (uint32_t)j) : 0;
 #pragma unroll
 			for (int o = 8; o > 0; o >>= 1) {
@@ -656,9 +665,9 @@ __global__ __launch_bounds__(256) void k_gemv_head(GemmArgs g) {
 		++it;
 	}
 	__syncthreads();
-	for (int q = threadIdx.x; q < it * MB * 16; q += 256) {
+	for (int q = threadIdx.x; q < it * MB * 16; q += 64 * NW) {
 		const int k = q / (MB * 16), tk = q % (MB * 16);
-		if (tk < g.M) e.argmax_key[(size_t)tk * e.key_ld + (int)blockIdx.x + k * (int)gridDim.x] = s_key[k][tk];
+		if (tk < M) e.argmax_key[(size_t)(m0 + tk) * e.key_ld + (int)blockIdx.x + k * (int)gridDim.x] = s_key[k][tk];
 	}
 }
 
@@ -765,7 +774,7 @@ __global__ __launch_bounds__(256) void k_gemv_w(GemmArgs g, int cps) {
 }
 
 // ------------------------------------------------------------------------------------------
-// Decode GEMVs on the packed weight layout (M <= 32).  Each projection keeps, beside its
+// Decode GEMVs on the packed weight layout (M <= 128, see kPkMaxM).  Each projection keeps, beside its
 // row-major matrix (read by the prefill GEMMs), a decode copy stored tile-major: for 16-column
 // tile t, 128-byte K chunk c and half h, the 1 KB block at ((t * C + c) * 2 + h) * 1024 holds,
 // for lane l = 16 grp + ri, the 16 bytes W[16 t + ri][128 c + 64 h + 16 grp .. +16) (rows past N
@@ -808,11 +817,13 @@ enum PkEpi { kPkRaw = 0, kPkFunnel = 1, kPkGeneral = 2 };
 // finishes token row w % 4 of row group w / 4.
 template <int MB, int NT, int CPW, int EPI, int NW = kGemvWaves>
 __global__ __launch_bounds__(64 * NW) void k_gemv_pk(GemmArgs g) {
-	static_assert(NW == kGemvWaves || (NW == 2 * kGemvWaves && MB == 2), "eight waves only for two row groups");
+	static_assert(NW == kGemvWaves || (NW == 2 * kGemvWaves && MB % 2 == 0), "eight waves share the row groups evenly");
 	__shared__ v4i red[2][NW][MB][64];
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ri = lane & 15, grp = lane >> 4;
 	const int C = g.K >> 7, T = (g.N + 15) / 16;
 	const v4i z = v4i{0, 0, 0, 0};
+	// this block's first token, and the tokens from it (row blocks: launches past 64 tokens)
+	const int m0 = MB == 4 ? blockIdx.y * (MB * 16) : 0, M = g.M - m0;
 	// the first tile's weights go out first: they need only wp, K and N
 	// a tile's weights, and its column's fold parameters, bias and segment fields, all fetched two
 	// tiles ahead so that no epilogue waits on a load
@@ -839,8 +850,8 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_pk(GemmArgs g) {
 #pragma unroll
 	for (int mb = 0; mb < MB; ++mb) {
 		const int r = mb * 16 + ri;
-		const bool rok = r < g.M;
-		const int8_t* arow = g.a + (size_t)(rok ? r : g.M - 1) * g.lda + grp * 16;
+		const bool rok = r < M;
+		const int8_t* arow = g.a + (size_t)(m0 + (rok ? r : M - 1)) * g.lda + grp * 16;
 #pragma unroll
 		for (int i = 0; i < CPW; ++i) {
 			const int c = wave * CPW + i;
@@ -879,7 +890,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_pk(GemmArgs g) {
 	const Scale* const in_scale = e.in_scale;
 #pragma unroll
 	for (int mb = 0; mb < MB; ++mb) {
-		const int tk = min(mb * 16 + grp * 4 + (wave & 3), g.M - 1);
+		const int tk = m0 + min(mb * 16 + grp * 4 + (wave & 3), M - 1);
 		p_rcp[mb] = EPI == kPkGeneral ? *(in_recip ? in_recip + tk : (const int64_t*)wp) : 0;
 		p_ein[mb] = EPI == kPkGeneral ? (in_scale ? in_scale + tk : (const Scale*)wp)->e : 0;
 	}
@@ -916,11 +927,12 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_pk(GemmArgs g) {
 		const int jj = j - sg.n_begin;
 #pragma unroll
 		for (int mb = 0; mb < MB; ++mb) {
-			if (NW != kGemvWaves && mb != (wave >> 2)) continue;  // (wave-uniform)
+			if (NW != kGemvWaves && (mb & 1) != (wave >> 2)) continue;  // (wave-uniform)
+			if (MB > 2 && mb * 16 >= M) continue;  // a row group past M (block-uniform)
 			int32_t tot = 0;
 #pragma unroll
 			for (int w = 0; w < NW; ++w) tot += ((const int32_t*)&red[i & 1][w][mb][lane])[wave & 3];
-			const int tk = mb * 16 + grp * 4 + (wave & 3);
+			const int tk = m0 + mb * 16 + grp * 4 + (wave & 3);
 			const bool live = col_ok && tk < g.M;
 			if (EPI == kPkRaw) {
 				if (live) raw_out[(size_t)tk * g.N + j] = tot;
@@ -966,6 +978,8 @@ __global__ __launch_bounds__(64 * WPB) void k_gemv_sk(GemmArgs g, int cps) {
 	const int C = g.K >> 7, T = (g.N + 15) / 16, split = blockIdx.y;
 	const int c0 = split * cps, c1 = min(C, c0 + cps);
 	const int tile0 = blockIdx.x * NTB;
+	// this block's first token, and the tokens from it (row blocks: launches past 64 tokens)
+	const int m0 = MB == 4 ? blockIdx.z * (MB * 16) : 0, M = g.M - m0;
 	for (int i = threadIdx.x; i < NTB * MB * 256; i += 64 * WPB) (&sum[0][0][0])[i] = 0;
 	__syncthreads();
 	const v4i z = v4i{0, 0, 0, 0};
@@ -984,8 +998,8 @@ __global__ __launch_bounds__(64 * WPB) void k_gemv_sk(GemmArgs g, int cps) {
 #pragma unroll
 	for (int mb = 0; mb < MB; ++mb) {
 		const int r = mb * 16 + ri;
-		const bool rok = r < g.M;
-		const int8_t* arow = g.a + (size_t)(rok ? r : g.M - 1) * g.lda + grp * 16;
+		const bool rok = r < M;
+		const int8_t* arow = g.a + (size_t)(m0 + (rok ? r : M - 1)) * g.lda + grp * 16;
 #pragma unroll
 		for (int i = 0; i < CPW; ++i) {
 			const int c = c0 + wave * CPW + i;
@@ -1014,7 +1028,7 @@ __global__ __launch_bounds__(64 * WPB) void k_gemv_sk(GemmArgs g, int cps) {
 	for (int i = threadIdx.x; i < NTB * MB * 256; i += 64 * WPB) {
 		const int t = i / (MB * 256), rem = i - t * MB * 256, tk = rem >> 4, col = rem & 15;
 		const int j = (tile0 + t) * 16 + col;
-		if (tk < g.M && j < g.N) plane[(size_t)tk * g.N + j] = sum[t][tk][col];
+		if (tk < M && j < g.N) plane[(size_t)(m0 + tk) * g.N + j] = sum[t][tk][col];
 	}
 }
 
@@ -4234,7 +4248,18 @@ void pack_gemv(const int8_t* w, int N, int K, int8_t* wp, hipStream_t s) {
 	hipLaunchKernelGGL(k_pack_gemv, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, w, N, K, wp, units);
 }
 
-constexpr int kPkMaxM = 32;  // two 16-token row groups
+// M <= 64: up to four 16-token row groups in one block; against the row-major k_gemv, 1.5B decode
+// layers + head at 64 tokens 4.1 -> 3.3 ms a step (50-request burst 216 -> 192 ms), 7B (4 layers) 2.02 ->
+// 1.64 ms.  M in 65..128: two row blocks of 64 side by side, each streaming the weights (the second
+// from the XCD's L2), where a wave holds its chunks of 64 activation rows beside the weights
+// (K <= 2048): a 96-token 1.5B prompt 3.25 -> 2.94 ms, 72 sequences 273 -> 250 ms a burst.  At
+// K = 3584 one eight-wave block fills a CU, the row blocks run one after the other and the 128-row
+// GEMM tiles win (7B, 100 sequences: 115 against 119 ms; 128-token prompts 7.8 against 9.1 ms).
+constexpr int kPkMaxM = 128;
+constexpr int kPkRowBlockMaxK = 2048;
+// k_gemv_sk's second row block at up to 2 chunks a wave (K <= 16,384): at the 7B down projection (3)
+// it loses too (100 sequences 114.4 -> 116.6 ms)
+constexpr int kSkRowBlockMaxCpw = 2;
 constexpr int kSkWaves = 8;
 
 // tiles per block of k_gemv_pk: the smallest instance >= an even share over the CUs
@@ -4243,12 +4268,6 @@ static int pk_nt(int T) {
 	for (int nt : {1, 2, 3, 5, 10})
 		if (nt >= need) return nt;
 	return 0;
-}
-
-// k_gemv_pk takes a launch without split planes or argmax keys at M <= 32, K <= 4096
-static bool pk_ok(const GemmArgs& g) {
-	return g.wp && g.M >= 1 && g.M <= kPkMaxM && g.K % 128 == 0 && g.K <= 4096 && !g.epi.argmax_key &&
-	       g.splits <= 1 && pk_nt((g.N + 15) / 16) > 0;
 }
 
 struct SkPlan {
@@ -4270,16 +4289,22 @@ static SkPlan sk_plan(int N, int K) {
 	return p;
 }
 
-static bool sk_ok(int M, int K, const GemmArgs* g) {
-	return M >= 1 && M <= kPkMaxM && K % 128 == 0 && K > 4096 && (!g || g->wp) && sk_plan(1, K).cpw > 0;
+int packed_planes(int M, int N, int K) {
+	if (M < 1 || M > kPkMaxM || K % 128) return 0;
+	if (K <= 4096) return (M <= 64 || K <= kPkRowBlockMaxK) && pk_nt((N + 15) / 16) > 0 ? 1 : 0;
+	const SkPlan p = sk_plan(N, K);  // splits 0: no instance
+	return M <= 64 || p.cpw <= kSkRowBlockMaxCpw ? p.splits : 0;
+}
+
+// k_gemv_pk takes a launch without split planes or argmax keys at K <= 4096
+static bool pk_ok(const GemmArgs& g) {
+	return g.wp && g.splits <= 1 && !g.epi.argmax_key && g.K <= 4096 && packed_planes(g.M, g.N, g.K) == 1;
 }
 
 int gemv_raw_splits(const GemmArgs& g) {
-	if (g.wp && g.M <= kPkMaxM && !g.epi.argmax_key && gemv_eligible(g.M, g.K)) {
-		if (g.K <= 4096 && pk_nt((g.N + 15) / 16) > 0) return 1;
-		if (sk_ok(g.M, g.K, &g)) return sk_plan(g.N, g.K).splits;
-	}
-	return gemv_plan(g.M, g.N, g.K, true, true).splits;
+	const int pk = g.wp && !g.epi.argmax_key ? packed_planes(g.M, g.N, g.K) : 0;
+	if (pk > 0) return pk;
+	return gemv_eligible(g.M, g.K) ? gemv_plan(g.M, g.N, g.K, true, true).splits : 0;
 }
 
 // chunks per wave of the k_gemv_pk instances: the smallest >= ceil(C / 4) (a larger one loads the
@@ -4302,25 +4327,42 @@ static int pk_epi(const GemmArgs& g) {
 }
 
 template <int MB, int NT, int EPI>
-static bool launch_pk_nt(const GemmArgs& g, int grid, int cpw, hipStream_t s) {
+static bool launch_pk_nt(const GemmArgs& g, int tile_blocks, int cpw, hipStream_t s) {
+	const dim3 grid(tile_blocks, (g.M + MB * 16 - 1) / (MB * 16));
+	if constexpr (MB == 4) {
+		// four row groups: activations of more than four chunks per wave would not stay in registers
+		switch (cpw) {
+#define X(W) \
+	case W: hipLaunchKernelGGL((k_gemv_pk<MB, NT, W, EPI>), grid, dim3(256), 0, s, g); return true;
+			X(1) X(2) X(3) X(4)
+#undef X
+		}
+		if ((g.K / 128 + 7) / 8 > 4) return false;
+		hipLaunchKernelGGL((k_gemv_pk<MB, NT, 4, EPI, 2 * kGemvWaves>), grid, dim3(64 * 2 * kGemvWaves), 0, s, g);
+		return true;
+	} else {
 	if constexpr (MB == 2 && NT >= 5) {
 		// two row groups over more than 16 chunks and several tiles per block: eight waves of 4
 		// (7B gate|up at M = 32: 30.5 -> 29.1 us; with 2-3 tiles per block, q|k|v and o, the
 		// larger block's fixed costs lost more: 8.6 -> 9.6 and 6.8 -> 7.5 us)
 		if (cpw > 4) {
 			if ((g.K / 128 + 7) / 8 > 4) return false;
-			hipLaunchKernelGGL((k_gemv_pk<MB, NT, 4, EPI, 2 * kGemvWaves>), dim3(grid), dim3(64 * 2 * kGemvWaves), 0, s, g);
+			hipLaunchKernelGGL((k_gemv_pk<MB, NT, 4, EPI, 2 * kGemvWaves>), grid, dim3(64 * 2 * kGemvWaves), 0, s, g);
 			return true;
 		}
 	}
 	switch (cpw) {
 #define X(W) \
-	case W: hipLaunchKernelGGL((k_gemv_pk<MB, NT, W, EPI>), dim3(grid), dim3(256), 0, s, g); return true;
+	case W: hipLaunchKernelGGL((k_gemv_pk<MB, NT, W, EPI>), grid, dim3(256), 0, s, g); return true;
 		X(1) X(2) X(3) X(4) X(7) X(8)
 #undef X
 	}
 	return false;
+	}
 }
+
+// 16-token row groups of a packed-GEMV instance: 1, 2 or 4
+static int pk_groups(int M) { return M <= 16 ? 1 : (M <= 32 ? 2 : 4); }
 
 template <int MB, int NT>
 static bool launch_pk_epi(const GemmArgs& g, int grid, int cpw, hipStream_t s) {
@@ -4334,10 +4376,12 @@ static bool launch_pk_epi(const GemmArgs& g, int grid, int cpw, hipStream_t s) {
 static bool launch_gemv_pk(const GemmArgs& g, hipStream_t s) {
 	const int T = (g.N + 15) / 16, C = g.K / 128;
 	const int nt = pk_nt(T), grid = (T + nt - 1) / nt, cpw = pk_cpw(C);
-	const bool two = g.M > 16;
+	const int mb = pk_groups(g.M);
 	switch (nt) {
 #define X(N) \
-	case N: return two ? launch_pk_epi<2, N>(g, grid, cpw, s) : launch_pk_epi<1, N>(g, grid, cpw, s);
+	case N: \
+		return mb == 1 ? launch_pk_epi<1, N>(g, grid, cpw, s) \
+		               : (mb == 2 ? launch_pk_epi<2, N>(g, grid, cpw, s) : launch_pk_epi<4, N>(g, grid, cpw, s));
 		X(1) X(2) X(3) X(5) X(10)
 #undef X
 	}
@@ -4346,7 +4390,7 @@ static bool launch_gemv_pk(const GemmArgs& g, hipStream_t s) {
 
 template <int MB, int NTB>
 static bool launch_sk_ntb(const GemmArgs& g, const SkPlan& p, hipStream_t s) {
-	const dim3 grid(p.bx, p.splits), block(64 * kSkWaves);
+	const dim3 grid(p.bx, p.splits, (g.M + MB * 16 - 1) / (MB * 16)), block(64 * kSkWaves);
 	switch (p.cpw) {
 #define X(W) \
 	case W: hipLaunchKernelGGL((k_gemv_sk<MB, NTB, W, kSkWaves>), grid, block, 0, s, g, p.cps); return true;
@@ -4360,36 +4404,45 @@ static bool launch_gemv_sk(const GemmArgs& g, hipStream_t s) {
 	const SkPlan p = sk_plan(g.N, g.K);
 	// the caller sized its planes by gemv_raw_splits(): a launch with another count is refused
 	if (p.cpw == 0 || g.splits != p.splits || !g.split_part) throw LaunchRefused{"gemv_sk: split count"};
-	const bool two = g.M > 16;
+	const int mb = pk_groups(g.M);
 	switch (p.ntb) {
 #define X(N) \
-	case N: return two ? launch_sk_ntb<2, N>(g, p, s) : launch_sk_ntb<1, N>(g, p, s);
+	case N: \
+		return mb == 1 ? launch_sk_ntb<1, N>(g, p, s) \
+		               : (mb == 2 ? launch_sk_ntb<2, N>(g, p, s) : launch_sk_ntb<4, N>(g, p, s));
 		X(1) X(2) X(3) X(4) X(6) X(7) X(8)
 #undef X
 	}
 	return false;
 }
 
-// k_gemv_head takes LM-head launches (argmax keys, no raw output) on the packed copy at M <= 32,
-// K <= 4096 (at most 8 chunks per wave); SSLM_HIP_HEAD_PK=0 keeps them on the generic GEMVs
+// k_gemv_head takes LM-head launches (argmax keys, no raw output) on the packed copy at the
+// sizes of kPkMaxM, K <= 4096 (at most 8 chunks per wave); SSLM_HIP_HEAD_PK=0 keeps them on the generic GEMVs
 static bool head_pk_ok(const GemmArgs& g) {
 	static const bool on = [] {
 		const char* e = getenv("SSLM_HIP_HEAD_PK");
 		return !(e && atoi(e) == 0);
 	}();
-	return on && g.wp && g.epi.argmax_key && !g.epi.raw_out && g.splits <= 1 && g.M >= 1 && g.M <= 32 &&
-	       g.K % 128 == 0 && g.K <= 4096;
+	return on && g.wp && g.epi.argmax_key && !g.epi.raw_out && g.splits <= 1 && g.M >= 1 && g.M <= kPkMaxM &&
+	       g.K % 128 == 0 && g.K <= 4096 && (g.M <= 64 || g.K <= kPkRowBlockMaxK);
 }
 
 template <int MB>
 static bool launch_gemv_head(const GemmArgs& g, hipStream_t s) {
 	const int C = g.K / 128, need = (C + kGemvWaves - 1) / kGemvWaves, T = (g.N + 15) / 16;
-	const int grid = std::min(T, std::max(device_cus(), (T + kHeadMaxSteps - 1) / kHeadMaxSteps));
+	const dim3 grid(std::min(T, std::max(device_cus(), (T + kHeadMaxSteps - 1) / kHeadMaxSteps)),
+	                (g.M + MB * 16 - 1) / (MB * 16));
+	if constexpr (MB == 4) {
+		if (need <= 3) hipLaunchKernelGGL((k_gemv_head<MB, 3>), grid, dim3(256), 0, s, g);
+		else hipLaunchKernelGGL((k_gemv_head<MB, 4, 2 * kGemvWaves>), grid, dim3(64 * 2 * kGemvWaves), 0, s, g);
+		return true;
+	} else {
 	switch (need <= 3 ? 3 : (need <= 4 ? 4 : (need <= 7 ? 7 : 8))) {
-		case 3: hipLaunchKernelGGL((k_gemv_head<MB, 3>), dim3(grid), dim3(256), 0, s, g); return true;
-		case 4: hipLaunchKernelGGL((k_gemv_head<MB, 4>), dim3(grid), dim3(256), 0, s, g); return true;
-		case 7: hipLaunchKernelGGL((k_gemv_head<MB, 7>), dim3(grid), dim3(256), 0, s, g); return true;
-		default: hipLaunchKernelGGL((k_gemv_head<MB, 8>), dim3(grid), dim3(256), 0, s, g); return true;
+		case 3: hipLaunchKernelGGL((k_gemv_head<MB, 3>), grid, dim3(256), 0, s, g); return true;
+		case 4: hipLaunchKernelGGL((k_gemv_head<MB, 4>), grid, dim3(256), 0, s, g); return true;
+		case 7: hipLaunchKernelGGL((k_gemv_head<MB, 7>), grid, dim3(256), 0, s, g); return true;
+		default: hipLaunchKernelGGL((k_gemv_head<MB, 8>), grid, dim3(256), 0, s, g); return true;
+	}
 	}
 }
 
@@ -4397,10 +4450,11 @@ void gemm(const GemmArgs& g, hipStream_t s) {
 	if (g.M <= 0 || g.N <= 0) return;
 	check_gemm_outputs(g);
 	if (head_pk_ok(g)) {
-		if (g.M > 16 ? launch_gemv_head<2>(g, s) : launch_gemv_head<1>(g, s)) return;
+		const int mb = pk_groups(g.M);
+		if (mb == 1 ? launch_gemv_head<1>(g, s) : (mb == 2 ? launch_gemv_head<2>(g, s) : launch_gemv_head<4>(g, s))) return;
 	}
-	if (gemv_eligible(g.M, g.K) && g.wp && g.M <= kPkMaxM && !g.epi.argmax_key) {
-		if (g.splits > 1 && sk_ok(g.M, g.K, &g)) {
+	if (g.wp && !g.epi.argmax_key && packed_planes(g.M, g.N, g.K) > 0) {
+		if (g.splits > 1 && g.K > 4096) {
 			if (launch_gemv_sk(g, s)) return;
 		} else if (pk_ok(g)) {
 			if (launch_gemv_pk(g, s)) return;

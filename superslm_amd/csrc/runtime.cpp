@@ -34,6 +34,11 @@ constexpr int kMaxTokens = 512;      // tokens per launch sequence (prefill chun
 constexpr int kTracks = 4;           // concurrent token groups of one decode step
 constexpr int kTrackTokens = 128;    // tokens per launch on tracks 1..kTracks-1
 constexpr int kSlotCapacity = 1024;  // live sequences per model
+// A decode unit (at most kTrackTokens rows) takes the sliced SiLU at any size (1.5B, 72 and 128
+// sequences: a burst 250.5 -> 246.9, 386.6 -> 383.0 ms); a prefill span only while it is this short: 100
+// prompts of 4-12 tokens 295.4 -> 292.6 ms, while at 65 and 96 tokens one block per row is faster (8 prompts
+// 23.2 against 23.5 and 23.6 against 24.9 ms).
+constexpr int kSlicedActPrefillRows = 32;
 
 struct HipError {
 	hipError_t e;
@@ -588,8 +593,8 @@ RawIn split_raw(sslm_model m, Track& w, GemmArgs& g, bool allow_multi, bool allo
 	// epilogue on the row: in the GEMV the epilogue's stores and waits sit behind the weight
 	// stream.  A prefill GEMM keeps its own epilogue unless it splits K.  The flags say which
 	// raw consumers fit their register budget (several planes / one plane).
-	if (sslm_launch::gemv_eligible(g.M, g.K)) {
-		splits = allow_multi ? sslm_launch::gemv_raw_splits(g) : 1;
+	if (const int planes = sslm_launch::gemv_raw_splits(g)) {
+		splits = allow_multi ? planes : 1;
 		if (splits == 1 && !allow_single) return r;
 	} else {
 		if (!allow_multi || lora || !sslm_launch::prefill_mfma_k(g.K)) return r;
@@ -820,7 +825,7 @@ void run_layers(sslm_model m, Track& w, int M, StreamRef st, int l0, int l1, ssl
 		sslm_launch::rmsnorm(a, M, H, w.tok, m->status, l0, s);
 		ck(hipGetLastError());
 	}
-	const bool fused = decode && sslm_launch::gemv_eligible(M, H) && fused_attention_enabled();
+	const bool fused = decode && M <= kTrackTokens && H % 128 == 0 && fused_attention_enabled();
 	const bool dbg = dbg_on(m, M);
 	for (int l = l0; l < l1; ++l) {
 		const DevLayer& lw = m->layers[l];
@@ -995,9 +1000,9 @@ void run_layers(sslm_model m, Track& w, int M, StreamRef st, int l0, int l1, ssl
 				a.up_tap = dbg_tap(m, l, kDbgUp);
 			}
 			ProfScope p(s, kProfRow, 0, 0);
-			// decode rows: one block per (row, column slice) in two launches, instead of one
-			// block per row that leaves most CUs idle
-			if (decode && sslm_launch::mlp_act_sliced_ok(a)) sslm_launch::mlp_act_sliced(a, s);
+			// short launches: one block per (row, column slice) in two launches, instead of one
+			// block per row that leaves most CUs idle (see kSlicedActPrefillRows)
+			if ((decode || M <= kSlicedActPrefillRows) && sslm_launch::mlp_act_sliced_ok(a)) sslm_launch::mlp_act_sliced(a, s);
 			else sslm_launch::mlp_act(a, s);
 			ck(hipGetLastError());
 			if (dbg) dbg_gather(m, w, l, kDbgAct, w.act, w.act_scale, nullptr, I, M);
@@ -1267,14 +1272,15 @@ void alloc_track(sslm_model m, Track& w, int T, bool head) {
 				}
 				// a GEMV and the narrow prefill kernel are always raw
 				if (sp > 1 || gemv || narrow) elems = std::max(elems, (size_t)sp * rows * sh[0]);
+				elems = std::max(elems, (size_t)sslm_launch::packed_planes(rows, sh[0], sh[1]) * rows * sh[0]);
 			}
 		}
 		w.raw_part = elems ? dalloc<int32_t>(elems, &own) : nullptr;
 	}
 	for (int i = 0; i < 3; ++i) w.lora_u[i] = dalloc<int8_t>((size_t)T * kMaxRank, &own);
-	w.act_prod = w.prefill ? nullptr : dalloc<int32_t>((size_t)sslm_launch::kMaxSlicedActRows * I, &own);
-	w.act_maxpart = w.prefill ? nullptr : dalloc<uint32_t>((size_t)sslm_launch::kMaxActSlices * kPartLd, &own);
-	w.gu_scale = w.prefill ? nullptr : dalloc<Scale>((size_t)sslm_launch::kMaxSlicedActRows * 2, &own);
+	w.act_prod = dalloc<int32_t>((size_t)sslm_launch::kMaxSlicedActRows * I, &own);
+	w.act_maxpart = dalloc<uint32_t>((size_t)sslm_launch::kMaxActSlices * kPartLd, &own);
+	w.gu_scale = dalloc<Scale>((size_t)sslm_launch::kMaxSlicedActRows * 2, &own);
 	w.kv_stage = w.prefill ? dalloc<int8_t>((size_t)T * 2 * KVH, &own) : nullptr;
 	w.sat_stage = w.prefill ? dalloc<uint32_t>(T, &own) : nullptr;
 	// the per-token attention keeps its rows in global scratch when they exceed LDS; a prefill
@@ -1513,7 +1519,7 @@ bool build_device_model(sslm_model m, std::string* err) {
 		m->d_pages = dupload(pages, &own);
 	}
 	// Packed decode copies of every projection and the LM head (read by the decode GEMVs at
-	// M <= 32; the row-major matrices stay for the prefill GEMMs).  SSLM_HIP_PACKED=0 keeps the
+	// M <= 128; the row-major matrices stay for the prefill GEMMs).  SSLM_HIP_PACKED=0 keeps the
 	// decode GEMVs on the row-major matrices.
 	if (packed_enabled()) {
 		auto packed = [&](const int8_t* wt, int N, int K) -> int8_t* {
