@@ -268,7 +268,7 @@ sslm_status sslm_hip_gemm_i32(const int8_t* a, const int8_t* w, int32_t m, int32
  * capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the
  * reference.  Same arguments, kernels and results as sslm_hip_gemm_requant, plus `stream` (a
  * hipStream_t; null = the default stream).  It allocates nothing: its scratch (int32 fold
- * outputs, per-tile partial maxima, per-token routing and scales) is one file-scope device array
+ * outputs, per-tile partial maxima) is one file-scope device array
  * of sslm_hip_noalloc_scratch_bytes() bytes (about 21 MB) that each GPU holds until the process
  * ends.  Asynchronous on `stream`: the outputs are ready once the stream has drained.  Calls on
  * one GPU share that array, so calls that overlap on one GPU (other streams, other threads) race;

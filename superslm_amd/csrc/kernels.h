@@ -289,6 +289,10 @@ struct FunnelArgs {
 	int32_t layer;
 	int32_t* status;
 	int32_t* head_status;  // or null: attention-stage refusals to resolve into `status` first
+	// standalone GEMM entries: `in_const` is every row's incoming scale (tok and incoming unused) and
+	// status[t] of each row t is written, not read
+	bool standalone;
+	Scale in_const;
 };
 void funnel(const FunnelArgs& a, hipStream_t s);
 

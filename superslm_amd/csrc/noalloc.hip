@@ -1,8 +1,7 @@
 // The GEMM + requant entry point for callers that cannot allocate device memory (code under HIP
 // graph capture, tight serving loops, harnesses that forbid hipMalloc): the same kernels as
-// sslm_hip_gemm_requant, with their scratch -- the int32 fold outputs, the per-(16-column tile,
-// token) partial maxima, the per-token routing and incoming scales -- in one file-scope device
-// array instead of library allocations.
+// sslm_hip_gemm_requant, with their scratch -- the int32 fold outputs and the per-(16-column tile,
+// token) partial maxima -- in one file-scope device array instead of library allocations.
 #include <hip/hip_runtime.h>
 #include <stdio.h>
 
@@ -24,9 +23,7 @@ static_assert(kNaMaxM <= kPartLd, "the partial maxima hold kPartLd tokens per ti
 constexpr size_t kOffF = 0;                                                  // int32 [M, N]
 constexpr size_t kOffMx = kOffF + (size_t)kNaMaxM * kNaMaxN * 4;             // uint32 [tile * kPartLd + t]
 constexpr size_t kMxWords = (size_t)(kNaMaxN / 16 - 1) * kPartLd + kNaMaxM;  // highest index + 1
-constexpr size_t kOffTok = (kOffMx + kMxWords * 4 + 255) / 256 * 256;        // TokenInfo [M]
-constexpr size_t kOffIn = (kOffTok + kNaMaxM * sizeof(TokenInfo) + 255) / 256 * 256;  // Scale [M]
-constexpr size_t kScratchBytes = (kOffIn + kNaMaxM * sizeof(Scale) + 255) / 256 * 256;
+constexpr size_t kScratchBytes = (kOffMx + kMxWords * 4 + 255) / 256 * 256;
 
 // Each GPU the library runs on holds its own copy until the process ends.  Host code never uses
 // this name as an address: it takes the per-device pointer from hipGetSymbolAddress.
@@ -53,16 +50,6 @@ unsigned char* scratch_ptr() {
 	return (unsigned char*)g_scratch_ptr[dev];
 }
 
-// Per-token routing (slot t, position 0), the incoming scale, and a cleared status per token:
-// a kernel, so the call records no memset or host copy.
-__global__ void k_noalloc_setup(TokenInfo* tok, Scale* in, int32_t* status, int m, int64_t in_m, int64_t in_e) {
-	const int t = blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= m) return;
-	tok[t] = TokenInfo{0, t, 0};
-	in[t] = Scale{in_m, in_e};
-	status[t] = 0;
-}
-
 }  // namespace
 
 extern "C" {
@@ -85,11 +72,6 @@ sslm_status sslm_hip_gemm_requant_noalloc(const int8_t* a, const int8_t* w, cons
 	(void)hipGetLastError();  // an error left by an unrelated earlier call is not this call's
 	int32_t* f = (int32_t*)(base + kOffF);
 	uint32_t* mx = (uint32_t*)(base + kOffMx);
-	TokenInfo* tok = (TokenInfo*)(base + kOffTok);
-	Scale* in = (Scale*)(base + kOffIn);
-
-	hipLaunchKernelGGL(k_noalloc_setup, dim3((m + 255) / 256), dim3(256), 0, stream, tok, in, out_status, m, in_m, in_e);
-	if (hipGetLastError() != hipSuccess) return SSLM_HIP_LAUNCH_FAILED;
 	GemmArgs g{};
 	g.a = a;
 	g.w = w;
@@ -97,7 +79,6 @@ sslm_status sslm_hip_gemm_requant_noalloc(const int8_t* a, const int8_t* w, cons
 	g.N = n;
 	g.K = k;
 	g.lda = k;
-	g.epi.tok = tok;
 	g.epi.status = out_status;
 	g.epi.nseg = 1;
 	Segment& sg = g.epi.seg[0];
@@ -117,12 +98,12 @@ sslm_status sslm_hip_gemm_requant_noalloc(const int8_t* a, const int8_t* w, cons
 	sslm_launch::FunnelArgs fa{};
 	fa.M = m;
 	fa.N = n;
-	fa.tok = tok;
+	fa.standalone = true;
+	fa.in_const = Scale{in_m, in_e};
 	fa.f = f;
 	fa.ld_f = n;
 	fa.maxpart = mx;
 	fa.ntiles = n / 16;
-	fa.incoming = in;
 	fa.site = Scale{site_m, site_e};
 	fa.out = out_codes;
 	fa.out_scale = (Scale*)out_me;

@@ -2945,9 +2945,6 @@ struct StandaloneCtx {
 	size_t f_n = 0;
 	uint32_t* mx = nullptr;
 	size_t mx_n = 0;
-	TokenInfo* tok = nullptr;
-	Scale* in = nullptr;
-	int cap_m = 0;
 	std::mutex mu;
 };
 StandaloneCtx g_sa;
@@ -2964,14 +2961,6 @@ void sa_reserve(int m, int n) {
 		g_sa.mx = dalloc<uint32_t>((size_t)(n + 15) / 16 * kPartLd, &g_sa.owned);
 		g_sa.mx_n = n;
 	}
-	if (m > g_sa.cap_m) {
-		g_sa.tok = dalloc<TokenInfo>(m, &g_sa.owned);
-		g_sa.in = dalloc<Scale>(m, &g_sa.owned);
-		std::vector<TokenInfo> ti(m);
-		for (int t = 0; t < m; ++t) ti[t] = TokenInfo{0, t, 0};
-		ck(hipMemcpy(g_sa.tok, ti.data(), m * sizeof(TokenInfo), hipMemcpyHostToDevice));
-		g_sa.cap_m = m;
-	}
 }
 
 GemmArgs sa_args(const int8_t* a, const int8_t* w, int m, int n, int k) {
@@ -2982,7 +2971,6 @@ GemmArgs sa_args(const int8_t* a, const int8_t* w, int m, int n, int k) {
 	g.N = n;
 	g.K = k;
 	g.lda = k;
-	g.epi.tok = g_sa.tok;
 	return g;
 }
 }  // namespace
@@ -2996,9 +2984,6 @@ sslm_status sslm_hip_gemm_requant(const int8_t* a, const int8_t* w, const int32_
 	return guarded([&]() -> sslm_status {
 		std::lock_guard<std::mutex> lk(g_sa.mu);
 		sa_reserve(m, n);
-		std::vector<Scale> in(m, Scale{in_m, in_e});
-		ck(hipMemcpyAsync(g_sa.in, in.data(), m * sizeof(Scale), hipMemcpyHostToDevice, g_sa.stream));
-		ck(hipMemsetAsync(out_status, 0, (size_t)m * 4, g_sa.stream));
 		GemmArgs g = sa_args(a, w, m, n, k);
 		g.epi.status = out_status;
 		g.epi.nseg = 1;
@@ -3012,12 +2997,12 @@ sslm_status sslm_hip_gemm_requant(const int8_t* a, const int8_t* w, const int32_
 		sslm_launch::FunnelArgs fa{};
 		fa.M = m;
 		fa.N = n;
-		fa.tok = g_sa.tok;
+		fa.standalone = true;
+		fa.in_const = Scale{in_m, in_e};
 		fa.f = g_sa.f;
 		fa.ld_f = n;
 		fa.maxpart = g_sa.mx;
 		fa.ntiles = (n + 15) / 16;
-		fa.incoming = g_sa.in;
 		fa.site = Scale{site_m, site_e};
 		fa.out = out_codes;
 		fa.out_scale = (Scale*)out_me;
