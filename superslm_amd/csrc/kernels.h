@@ -204,7 +204,7 @@ struct QkvPostArgs {
 	uint32_t* sat_stage;
 };
 void qkv_post(const QkvPostArgs& a, hipStream_t s);
-// Writes the staged K/V rows of a prefill span into the pool and adds the clamp counts, unless
+// (unless tiled_attention_staged()) Writes the staged K/V rows of a prefill span into the pool and adds the clamp counts, unless
 // the slot's status holds a refusal; always clears sat_stage.
 void kv_commit(const QkvPostArgs& a, hipStream_t s);
 
@@ -243,6 +243,10 @@ struct AttnArgs {
 	SiteTap q_tap;              // attention_decode: the rotated q codes of each head, and the q scale
 	int32_t wcap;               // attention_decode: score rows of the grouped kernel, a multiple of 128
 	                            // at least every width (pos + 1) of the launch (group_width_cap)
+	// attention() where tiled_attention_staged(): the span's staged K/V rows and clamp counts
+	// (QkvPostArgs), which the kernel reads and commits to the pool and `sat`
+	const int8_t* kv_stage;
+	uint32_t* sat_stage;
 	int32_t row_halves;         // attention_decode, grouped kernel: 1, or 2 blocks per (token, KV group)
 };
 // The grouped decode kernel's score-row length for a launch whose widest row is `max_width`:
@@ -256,6 +260,9 @@ inline int32_t group_width_cap(int64_t max_width, int64_t cap) {
 // the query-tiled kernel may run (unless SSLM_HIP_TILED_ATTN=0).
 void attention(const AttnArgs& a, hipStream_t s, bool one_sequence = false);
 bool tiled_attention_enabled();
+// the span's query-tiled kernel reads staged K/V rows and commits them itself (8-wave blocks); else
+// kv_commit runs before the attention
+bool tiled_attention_staged(int M, int NKV, int NH);
 // Decode attention with the q|k|v post-processing fused in (one block per (query head, token)):
 // valid when every token of the launch belongs to a different sequence, so no token attends to
 // a position another block of the launch writes.

@@ -3269,6 +3269,15 @@ __global__ __launch_bounds__(BS) void k_attention(sslm_launch::AttnArgs a) {
 // below 2^22 in magnitude).  V rows are staged in LDS as stored ([position][dim]) and read with
 // gfx950's byte-transposing LDS load, so a lane's 16 B operand holds 16 positions of one dimension.
 // The launch must hold one sequence's consecutive positions (a prefill chunk).
+// 8-wave blocks (grids of less than two blocks per CU) read the span's own K/V rows from the staging
+// rows k_qkv_post left ([token][K heads | V heads][D]) and the earlier positions from the pool; the
+// first head of each KV group writes its tile's rows into the pool and adds the clamp counts, which
+// was a launch of its own between the two kernels (k_kv_commit, 4.0-4.8 us a layer).  No block reads
+// a pool row that another block of the launch writes.  The first step's K and V rows and the query
+// rows are issued at entry, under the derivation of the i-exp constants, and the first step keeps its
+// scores through the passes: a span of at most 128 positions reads K once (100 prompts of 4-12
+// tokens and their decoding 293.6 -> 280.4 ms).  4-wave blocks, held to 3 a CU, have no registers
+// for either (2,048-token 7B attention 321 -> 369 us with them): k_kv_commit runs before them.
 constexpr int kTiledECache = 512;  // positions whose i-exp values an 8-wave tiled-attention block keeps
 
 template <int D, int NW>
@@ -3299,7 +3308,47 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 	const int t0 = tile * TQ, nt = min(TQ, a.M - t0);
 	const int kvh = h / group;
 	const TokenInfo ti0 = a.tok[t0];
-	if (threadIdx.x == 0) s_st = a.status[ti0.slot];
+	const int span0 = (int)a.tok[0].pos, last = span0 + a.M - 1;  // the launch's positions
+	const int KVH = a.NKV * D;
+	const int8_t* kbase = a.kv_pool + (int64_t)ti0.block * a.block_bytes + (int64_t)a.layer * a.cap * KVH * 2 +
+	                      (int64_t)kvh * a.cap * D;
+	const int8_t* vbase = kbase + a.cap * (int64_t)KVH;
+	constexpr bool STAGED = NW == 8;
+	const int8_t* kstage = STAGED ? a.kv_stage + (int64_t)kvh * D : nullptr;
+	// K row of position p (past the launch's last: the last one); V rows lie KVH further in the
+	// staging rows and in the other half of the pool block
+	auto k_row = [&](int p) {
+		if (!STAGED) return kbase + (int64_t)min(p, (int)a.cap - 1) * D;
+		const int pc = min(p, last);
+		return pc >= span0 ? kstage + (int64_t)(pc - span0) * (2 * KVH) : kbase + (int64_t)pc * D;
+	};
+	auto v_row = [&](int p) {
+		if (!STAGED) return vbase + (int64_t)min(p, (int)a.cap - 1) * D;
+		const int pc = min(p, last);
+		return pc >= span0 ? kstage + KVH + (int64_t)(pc - span0) * (2 * KVH) : vbase + (int64_t)pc * D;
+	};
+	constexpr int VCH = KB * (D / 16), VPT = (VCH + 64 * NW - 1) / (64 * NW);  // V chunks per thread and step
+	// this lane's A operand: query row ri, bytes c*64 + g*16 of chunk c; then the first step's K and V
+	v4i qa[NC], k0r[NC], v0r[VPT];
+	const int st0 = a.status[ti0.slot];
+#pragma unroll
+	for (int c = 0; c < NC; ++c) {
+		const int off = min(c * 64 + g * 16, D - 16);
+		qa[c] = load16(a.q_rot + (size_t)(t0 + min(ri, nt - 1)) * a.H + (size_t)h * D + off);
+		if (STAGED) k0r[c] = load16(k_row(wave * 16 + ri) + off);
+	}
+#pragma unroll
+	for (int u = 0; u < VPT; ++u) {
+		const int c = min((int)threadIdx.x + u * 64 * NW, VCH - 1);
+		if (STAGED) v0r[u] = load16(v_row(c / (D / 16)) + (c % (D / 16)) * 16);
+	}
+#pragma unroll
+	for (int c = 0; c < NC; ++c) {
+		const bool off_ok = c * 64 + g * 16 < D;
+		qa[c] = ri < nt && off_ok ? qa[c] : v4i{0, 0, 0, 0};
+		if (STAGED) k0r[c] = off_ok ? k0r[c] : v4i{0, 0, 0, 0};
+	}
+	if (threadIdx.x == 0) s_st = st0;
 	if (threadIdx.x < TQ) {
 		// the token's i-exp constants and width, as k_attention derives them
 		const int tq = threadIdx.x;
@@ -3336,23 +3385,25 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 		s_rf[tq] = 0;
 	}
 	__syncthreads();
+	if (STAGED && h == 0 && threadIdx.x < nt) {  // the tile's clamp counts, cleared whatever the status
+		const uint32_t sat = a.sat_stage[t0 + threadIdx.x];
+		a.sat_stage[t0 + threadIdx.x] = 0;
+		if (s_st == 0 && sat) atomicAdd(&a.sat[ti0.slot], (unsigned long long)sat);
+	}
 	if (s_st != 0) return;
+	if (STAGED && h % group == 0) {  // the tile's K/V rows of this KV head, into the pool
+		for (int c = threadIdx.x; c < nt * (D / 8); c += 64 * NW) {
+			const int tq = c / (D / 8), r = c % (D / 8), kv = r / (D / 16), ch = r % (D / 16);
+			int8_t* dst = (int8_t*)(kv ? vbase : kbase) + (int64_t)(span0 + t0 + tq) * D + ch * 16;
+			*(v4i*)dst = load16(kstage + (int64_t)kv * KVH + (int64_t)(t0 + tq) * (2 * KVH) + ch * 16);
+		}
+	}
 	if (threadIdx.x < nt && s_ok[threadIdx.x] != kOk)
 		report_head(a.head_status, ti0.slot, h, s_ok[threadIdx.x] == -1 ? kPositionOverCap : s_ok[threadIdx.x]);
 	int wmax = 0;  // positions [0, wmax) cover every live token's row
 	for (int tq = 0; tq < nt; ++tq)
 		if (s_ok[tq] == kOk) wmax = max(wmax, s_pos[tq] + 1);
 	if (wmax == 0) return;
-	const int8_t* kbase = a.kv_pool + (int64_t)ti0.block * a.block_bytes + (int64_t)a.layer * a.cap * a.NKV * D * 2 +
-	                      (int64_t)kvh * a.cap * D;
-	const int8_t* vbase = kbase + a.cap * (int64_t)a.NKV * D;
-	// this lane's A operand: query row ri, bytes c*64 + g*16 of chunk c
-	v4i qa[NC];
-#pragma unroll
-	for (int c = 0; c < NC; ++c) {
-		const int off = c * 64 + g * 16;
-		qa[c] = ri < nt && off < D ? load16(a.q_rot + (size_t)(t0 + ri) * a.H + (size_t)h * D + off) : v4i{0, 0, 0, 0};
-	}
 	// the output tokens of this lane: g*4 + v
 	int32_t tpos[4];
 	bool tok_ok[4];
@@ -3365,7 +3416,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 	const bool ecache = NW == 8 && nblk * KB <= ECP;
 	auto scores = [&](int blk, int* p_out) {
 		const int p = blk * KB + wave * 16 + ri;
-		const int8_t* kr = kbase + (int64_t)min(p, (int)a.cap - 1) * D;
+		const int8_t* kr = k_row(p);
 		v4i acc = v4i{0, 0, 0, 0};
 #pragma unroll
 		for (int c = 0; c < NC; ++c) {
@@ -3376,9 +3427,17 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 		*p_out = p;
 		return acc;
 	};
+	v4i s0 = v4i{0, 0, 0, 0};  // the first step's scores, for every pass
+#pragma unroll
+	for (int c = 0; c < NC; ++c)
+		if (STAGED) s0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(qa[c], k0r[c], s0, 0, 0, 0);
+	const int p0 = wave * 16 + ri;
 	// pass 1: row maxima
 	int32_t mx[4] = {INT32_MIN, INT32_MIN, INT32_MIN, INT32_MIN};
-	for (int blk = 0; blk < nblk; ++blk) {
+#pragma unroll
+	for (int v = 0; v < 4; ++v)
+		if (STAGED && tok_ok[v] && p0 <= tpos[v]) mx[v] = s0[v];
+	for (int blk = STAGED ? 1 : 0; blk < nblk; ++blk) {
 		int p;
 		const v4i s = scores(blk, &p);
 #pragma unroll
@@ -3418,8 +3477,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 	int64_t sum[4] = {0, 0, 0, 0};
 	uint32_t refused = 0;
 	for (int blk = 0; blk < nblk; ++blk) {
-		int p;
-		const v4i s = scores(blk, &p);
+		int p = p0;
+		v4i s = s0;
+		if (!STAGED || blk > 0) s = scores(blk, &p);
 #pragma unroll
 		for (int v = 0; v < 4; ++v) {
 			if (tok_ok[v] && p <= tpos[v]) {
@@ -3465,20 +3525,19 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 #pragma unroll
 		for (int k = 0; k < 3; ++k) cacc[i][k] = v4i{0, 0, 0, 0};
 	// a step's V rows are issued before its probabilities are computed and stored to LDS after
-	// them (16-byte copies; rows past the cap repeat the last one)
-	constexpr int VCH = KB * (D / 16), VPT = (VCH + 64 * NW - 1) / (64 * NW);  // V chunks per thread
+	// them (16-byte copies; rows past the launch repeat its last one)
 	for (int blk = 0; blk < nblk; ++blk) {
 		v4i vr[VPT];
 #pragma unroll
 		for (int u = 0; u < VPT; ++u) {
 			const int c = min((int)threadIdx.x + u * 64 * NW, VCH - 1);
-			const int64_t pos = min(blk * KB + c / (D / 16), (int)a.cap - 1);
-			vr[u] = load16(vbase + pos * D + (c % (D / 16)) * 16);
+			if (STAGED) vr[u] = v0r[u];
+			if (!STAGED || blk > 0) vr[u] = load16(v_row(blk * KB + c / (D / 16)) + (c % (D / 16)) * 16);
 		}
-		int p;
-		v4i s = v4i{0, 0, 0, 0};
+		int p = p0;
+		v4i s = s0;
 		if (ecache) p = blk * KB + wave * 16 + ri;
-		else s = scores(blk, &p);
+		else if (!STAGED || blk > 0) s = scores(blk, &p);
 		const int pl = wave * 16 + ri;
 #pragma unroll
 		for (int v = 0; v < 4; ++v) {
@@ -4827,11 +4886,8 @@ void attention(const AttnArgs& a, hipStream_t s, bool one_sequence) {
 	}
 	const int groups = ((a.M + 15) / 16) * a.NKV, per_xcd = (groups + 7) / 8;
 	const dim3 grid(per_xcd * 8 * (a.NH / a.NKV));  // see the XCD-aware order in k_attention_tiled
-	// 8 waves (128 positions per step) halve the longest rows' serial chain when the grid is
-	// small; with two or more blocks per CU, 4-wave blocks pack the CUs better
-	// SSLM_HIP_TILED_WAVES=4 or 8 overrides the choice (read per launch; the parity tests run both)
-	const char* fw = getenv("SSLM_HIP_TILED_WAVES");
-	const bool wide = fw && fw[0] ? fw[0] == '8' : (int)grid.x < 2 * 256;  // MI355X: 256 CUs
+	const bool wide = tiled_attention_staged(a.M, a.NKV, a.NH);
+	if (wide && !(a.kv_stage && a.sat_stage && a.sat)) throw LaunchRefused{"tiled attention: no staged rows"};
 	switch (a.D) {
 		case 32: if (wide) hipLaunchKernelGGL((k_attention_tiled<32, 8>), grid, dim3(512), 0, s, a); else hipLaunchKernelGGL((k_attention_tiled<32, 4>), grid, dim3(256), 0, s, a); break;
 		case 64: if (wide) hipLaunchKernelGGL((k_attention_tiled<64, 8>), grid, dim3(512), 0, s, a); else hipLaunchKernelGGL((k_attention_tiled<64, 4>), grid, dim3(256), 0, s, a); break;
@@ -4839,6 +4895,16 @@ void attention(const AttnArgs& a, hipStream_t s, bool one_sequence) {
 		case 256: if (wide) hipLaunchKernelGGL((k_attention_tiled<256, 8>), grid, dim3(512), 0, s, a); else hipLaunchKernelGGL((k_attention_tiled<256, 4>), grid, dim3(256), 0, s, a); break;
 		default: no_instance("attention", a.D);
 	}
+}
+
+bool tiled_attention_staged(int M, int NKV, int NH) {
+	if (!tiled_attention_enabled()) return false;
+	const int groups = ((M + 15) / 16) * NKV, blocks = (groups + 7) / 8 * 8 * (NH / NKV);
+	// 8 waves (128 positions per step) halve the longest rows' serial chain when the grid is
+	// small; with two or more blocks per CU, 4-wave blocks pack the CUs better
+	// SSLM_HIP_TILED_WAVES=4 or 8 overrides the choice (read per launch; the parity tests run both)
+	const char* fw = getenv("SSLM_HIP_TILED_WAVES");
+	return fw && fw[0] ? fw[0] == '8' : blocks < 2 * 256;  // MI355X: 256 CUs
 }
 
 bool tiled_attention_enabled() {

@@ -826,6 +826,7 @@ void run_layers(sslm_model m, Track& w, int M, StreamRef st, int l0, int l1, ssl
 		ck(hipGetLastError());
 	}
 	const bool fused = decode && M <= kTrackTokens && H % 128 == 0 && fused_attention_enabled();
+	const bool staged_attn = !decode && w.kv_stage && sslm_launch::tiled_attention_staged(M, m->NKV, m->NH);
 	const bool dbg = dbg_on(m, M);
 	for (int l = l0; l < l1; ++l) {
 		const DevLayer& lw = m->layers[l];
@@ -894,7 +895,7 @@ void run_layers(sslm_model m, Track& w, int M, StreamRef st, int l0, int l1, ssl
 				ProfScope p(s, kProfRow, 0, 0);
 				sslm_launch::qkv_post(a, s);
 				ck(hipGetLastError());
-				if (a.kv_stage) {
+				if (a.kv_stage && !staged_attn) {
 					sslm_launch::kv_commit(a, s);
 					ck(hipGetLastError());
 				}
@@ -903,6 +904,11 @@ void run_layers(sslm_model m, Track& w, int M, StreamRef st, int l0, int l1, ssl
 			sslm_launch::AttnArgs aa = attn_args(m, w, l, M);
 			aa.q_rot = w.q_rot;
 			aa.q_scale = w.q_scale;
+			if (staged_attn) {  // the attention commits the span's K/V
+				aa.kv_stage = w.kv_stage;
+				aa.sat_stage = w.sat_stage;
+				aa.sat = m->sat;
+			}
 			ProfScope p(s, kProfAttn, 0, 0);
 			sslm_launch::attention(aa, s, !decode);  // prefill chunks: one sequence, consecutive positions
 			ck(hipGetLastError());
