@@ -221,23 +221,27 @@ SSLM_HD int8_t requant_code_small(int64_t x, uint64_t r, int s) {
 // requant_code_small in double arithmetic, for |x| <= 2^31 and a funnel plan's (r, s), r in
 // (2^31, 2^32] and s in [-1, 30].  The code is floor(q + 1/2), clamped to 127, for the exact
 // quotient q = |x| 127 r / 2^(62-s).  f = 127 r 2^-(62-s) is exact in a double (127 r < 2^39),
-// so |x| f is q rounded once and fma returns that rounding error exactly.  Rounding is
-// monotone, so m0 = floor(rounded q + 1/2) is the code or one more; it is one more exactly when
-// (rounded q - (m0 - 1/2)) + err < 0, a sign that is exact wherever it can be near zero
-// (Sterbenz: there the rounded q is within 2^-40 of m0 - 1/2 >= 1/2).  Every operation is full
-// rate on CDNA's FP64 pipes, where the 128-bit integer form takes eight quarter-rate multiplies.
+// so q = |x| f exactly and fma(|x|, f, 1/2) is q + 1/2 rounded once.  Rounding is monotone, so
+// m0 = floor of it is the code or, where q + 1/2 was rounded up to an integer, one more; that is
+// exactly when |x| f + (1/2 - m0) < 0, and an fma has the sign of its exact value (1/2 - m0 is exact
+// for every m0 that can be a code).  Every operation is full rate on CDNA's FP64 pipes, where the
+// 128-bit integer form takes eight quarter-rate multiplies.
 SSLM_HD double requant_factor(int64_t r, int s) { return ldexp((double)(r * 127), -(62 - s)); }
+SSLM_HD int32_t requant_mag(double a, double f) {  // a = |x|
+	const double m0 = floor(fma(a, f, 0.5));
+	const double e = fma(a, f, 0.5 - m0);
+	const int32_t c = (int32_t)fmin(m0, 128.0) - (e < 0.0 ? 1 : 0);
+	return c > 127 ? 127 : c;
+}
 SSLM_HD int8_t requant_code_f(int64_t x, double f) {
-#pragma clang fp contract(off)
 	const uint32_t ax = x < 0 ? 0u - (uint32_t)x : (uint32_t)x;
-	const double a = (double)ax;
-	const double qh = a * f;
-	const double er = fma(a, f, -qh);
-	const double q = fmin(qh, 255.0);  // past 255 the code saturates whatever the error
-	const double m0 = floor(q + 0.5);
-	const double m = (q - (m0 - 0.5)) + er < 0.0 ? m0 - 1.0 : m0;
-	const int32_t c = (int32_t)fmin(m, 127.0);
+	const int32_t c = requant_mag((double)ax, f);
 	return (int8_t)(x < 0 ? -c : c);
+}
+// the same for an integral double x
+SSLM_HD int8_t requant_code_d(double x, double f) {
+	const int32_t c = requant_mag(fabs(x), f);
+	return (int8_t)(x < 0.0 ? -c : c);
 }
 
 // src/intmath.cpp:502-524
@@ -708,23 +712,16 @@ SSLM_HD int32_t div_q15_small(int64_t e, double d, double inv) {
 
 // floor(v 2^32 / root) for a code v in [-128, 127] and 1 <= root < 2^24 (the RMSNorm's
 // per-code quotient, forward_sites.cpp:410-459: floor for v >= 0, -ceil(|v| 2^32 / root) below),
-// given inv = 1.0 / root.  n = |v| 2^32 <= 2^39 is exact in a double and the estimate n inv is
-// within one of the quotient; q root <= n + root < 2^53 is exact too, so fma gives the exact
+// given inv = 1.0 / root.  n = v 2^32 (|n| <= 2^39) is exact in a double and the estimate n inv is
+// within 2^-12 of the quotient; q root <= |n| + root < 2^53 is exact too, so fma gives the exact
 // remainder for the one-step correction.
-SSLM_HD int64_t norm_fd(int32_t v, double root, double inv) {
-	const double n = ldexp((double)(v < 0 ? -v : v), 32);
-	double q = floor(n * inv);
-	double r = fma(-q, root, n);
-	if (r < 0.0) {
-		q -= 1.0;
-		r += root;
-	} else if (r >= root) {
-		q += 1.0;
-		r -= root;
-	}
-	const int64_t qi = (int64_t)q;
-	return v >= 0 ? qi : -(qi + (r > 0.0 ? 1 : 0));
+SSLM_HD double norm_qd(int32_t v, double root, double inv) {
+	const double n = (double)v * 4294967296.0;
+	const double q = floor(n * inv);
+	const double r = fma(-q, root, n);
+	return r < 0.0 ? q - 1.0 : (r >= root ? q + 1.0 : q);
 }
+SSLM_HD int64_t norm_fd(int32_t v, double root, double inv) { return (int64_t)norm_qd(v, root, inv); }
 
 SSLM_HD int64_t softmax_ceiling(int64_t q_b, int64_t q_c) {
 	s128 m128 = (s128)q_b * q_b + (s128)q_c;

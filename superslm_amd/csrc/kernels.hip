@@ -72,6 +72,9 @@ __device__ __forceinline__ uint32_t sat_abs_u32(int64_t v) {
 	return a > 0xfffffffeull ? 0xfffffffeu : (uint32_t)a;
 }
 
+// sat_abs_u32 of a row maximum held in a non-negative double
+__device__ __forceinline__ uint32_t sat_u32_d(double m) { return (uint32_t)fmin(m, 4294967294.0); }
+
 // The row of a one-block-per-row launch: workgroups go to the 8 XCDs in turn (block b on XCD
 // b % 8), so giving each XCD a contiguous run of rows keeps a tile-major maxima array's lines
 // ([tile][row], 32 rows to a line) in one XCD's L2 instead of fetched by all eight.  Identity
@@ -2122,23 +2125,23 @@ __device__ __forceinline__ int32_t rmsnorm_regs(const int32_t (&h)[EPT], const i
 	// floor((v << 32) / root) per element from one shared reciprocal (root < 2^23)
 	const double rd = (double)root, inv = 1.0 / rd;
 	KT(11);
-	int64_t w[EPT];
-	uint32_t mx = 0;
+	double w[EPT], mxd = 0.0;  // |quotient * gain| < 2^39 * 2^7: exact in doubles
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) {
-		w[k] = norm_fd(h[k], rd, inv) * (int64_t)g[k];
-		mx = max(mx, sat_abs_u32(w[k]));
+		w[k] = norm_qd(h[k], rd, inv) * (double)g[k];
+		mxd = fmax(mxd, fabs(w[k]));
 	}
-	mx = blk_max32<BS>(mx, s_max);
+	const uint32_t mx = blk_max32<BS>(sat_u32_d(mxd), s_max);
 	KT(12);
 	FunnelPlan plan;
 	const int32_t st = funnel_plan(mx, nullptr, 0, site, &plan);
 	if (st != kOk) return st;
 	KT(13);
+	const double f = requant_factor(plan.r, plan.s);
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) {
 		const int i = threadIdx.x + k * BS;
-		if (i < H) out[i] = requant_code_f(w[k], requant_factor(plan.r, plan.s));
+		if (i < H) out[i] = requant_code_d(w[k], f);
 	}
 	if (threadIdx.x == 0) {
 		*out_scale = plan.out;
@@ -2515,7 +2518,7 @@ template <int BS, int EPT, int RS>
 __global__ __launch_bounds__(BS) void k_residual_norm(sslm_launch::ResidualArgs a) {
 	__shared__ uint32_t s_b[BS / 64], s_r[BS / 64], s_n[BS / 64];
 	__shared__ int32_t s_ss[BS / 64];
-	__shared__ int64_t land[256];  // landed branch value per branch code (code + 127)
+	__shared__ double land[256];  // landed branch value per branch code (code + 127)
 	__shared__ int32_t s_st;
 	const int t = blockIdx.x, H = a.H;
 	KT(0);
@@ -2540,21 +2543,40 @@ __global__ __launch_bounds__(BS) void k_residual_norm(sslm_launch::ResidualArgs 
 	}
 	uint32_t bmx = 0;
 	if (RS > 0) {
-		int j[EPT];
-		bool live[EPT];
-		int64_t v[EPT];
+		// as raw_row, without a bias (the o and down projections have none): the bounded fold keeps the
+		// values in int32 (|acc| <= 127 * 128 * K < 2^29), an adapter's delta widens them
+		const Segment& sg = a.raw.epi.seg[0];
+		const size_t plane = (size_t)a.M * a.raw.ld;
+		const int32_t* row = a.raw.part + (size_t)t * a.raw.ld;
+		uint32_t acc[EPT];
+		int32_t f0[EPT], f1[EPT], f2[EPT];
 #pragma unroll
 		for (int k = 0; k < EPT; ++k) {
-			j[k] = threadIdx.x + k * BS;
-			live[k] = j[k] < H;
+			const int jc = min((int)threadIdx.x + k * BS, H - 1);
+			acc[k] = 0;
+#pragma unroll
+			for (int s2 = 0; s2 < RS; ++s2) {  // clamped plane index: no branch, no extra round trip
+				const uint32_t x = (uint32_t)row[(size_t)(RS == 1 ? 0 : min(s2, a.raw.splits - 1)) * plane + jc];
+				acc[k] += (RS == 1 || s2 < a.raw.splits) ? x : 0u;
+			}
+			const int32_t* f = sg.fold + 3 * jc;
+			f0[k] = f[0];
+			f1[k] = f[1];
+			f2[k] = f[2];
 		}
-		const bool ok = raw_row<EPT, RS>(a.raw, 0, a.M, t, j, live, v);
 #pragma unroll
 		for (int k = 0; k < EPT; ++k) {
-			bf[k] = sat_i32(v[k]);
-			bmx = max(bmx, sat_abs_u32(v[k]));
+			const bool in = (int)threadIdx.x + k * BS < H;
+			const int32_t v = fold_bounded((int32_t)acc[k], fold_consts(f0[k], f1[k], f2[k]));
+			bf[k] = in ? v : 0;
+			uint32_t m = (uint32_t)(bf[k] < 0 ? -bf[k] : bf[k]);
+			if (sg.lora_b && in) {
+				const int64_t vl = (int64_t)v + lora_delta(sg, a.raw.epi.rank, t, (int)threadIdx.x + k * BS);
+				bf[k] = sat_i32(vl);
+				m = sat_abs_u32(vl);
+			}
+			bmx = max(bmx, m);
 		}
-		if (!ok) bmx = kBad32;
 	}
 	if (RS == 0) load_row<BS>(bfr, H, bf);
 	if (RS == 0) bmx = part_max32_fixed<BS, (EPT + 15) / 16>(a.branch_maxpart, 0, H / 16, t);
@@ -2563,7 +2585,7 @@ __global__ __launch_bounds__(BS) void k_residual_norm(sslm_launch::ResidualArgs 
 	KT(1);
 	if (s_st != 0) return;
 	FunnelPlan bplan;
-	int32_t st = bmx == kBad32 ? kBiasReconcileProductOutOfDomain : funnel_plan(bmx, &bin, 1, a.branch_site, &bplan);
+	int32_t st = funnel_plan(bmx, &bin, 1, a.branch_site, &bplan);
 	if (st == kOk && !fits_i32(ss.m)) st = kCarriedScaleMantissaOutOfDomain;
 	if (st != kOk) {
 		if (threadIdx.x == 0) set_status(a.status, slot, a.layer, st);
@@ -2572,10 +2594,12 @@ __global__ __launch_bounds__(BS) void k_residual_norm(sslm_launch::ResidualArgs 
 	KT(2);
 	// The landed value depends on the branch code alone (forward_sites.cpp:513-653 with the
 	// row's scales fixed), so the 255 possible values are tabulated, one per thread;
-	// INT64_MIN marks a code whose landing exceeds int64.
+	// infinity marks a code whose landing exceeds int64.  Doubles hold every value the residual funnel
+	// accepts (at most 2^31) exactly.
 	int32_t code[EPT];
+	const double bfac = requant_factor(bplan.r, bplan.s);
 #pragma unroll
-	for (int k = 0; k < EPT; ++k) code[k] = requant_code_f(bf[k], requant_factor(bplan.r, bplan.s));
+	for (int k = 0; k < EPT; ++k) code[k] = requant_code_f(bf[k], bfac);
 	if (a.branch_tap.codes) {
 #pragma unroll
 		for (int k = 0; k < EPT; ++k) {
@@ -2589,26 +2613,16 @@ __global__ __launch_bounds__(BS) void k_residual_norm(sslm_launch::ResidualArgs 
 		const int64_t kx = composed_exponent(bplan.out.e, ss.e);
 		bool cl, ex;
 		const int64_t rec = landing_small((int64_t)threadIdx.x - 127, bplan.out.m, r_h, kx, &cl, &ex);
-		land[threadIdx.x] = ex ? kI64Min : rec;
+		land[threadIdx.x] = ex ? (double)INFINITY : (double)rec;
 	}
 	__syncthreads();
-	int64_t w[EPT];
-	uint32_t mx = 0;
+	double w[EPT], mxd = 0.0;
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) {
-		const int i = threadIdx.x + k * BS;
-		w[k] = 0;
-		if (i < H) {
-			const int64_t rec = land[code[k] + 127];
-			if (rec == kI64Min) {
-				mx = kBad32;
-			} else {
-				w[k] = rec + sv[k];
-				mx = max(mx, sat_abs_u32(w[k]));
-			}
-		}
+		w[k] = (int)threadIdx.x + k * BS < H ? land[code[k] + 127] + (double)sv[k] : 0.0;
+		mxd = fmax(mxd, fabs(w[k]));
 	}
-	mx = blk_max32<BS>(mx, s_r);
+	const uint32_t mx = blk_max32<BS>(mxd == (double)INFINITY ? kBad32 : sat_u32_d(mxd), s_r);
 	KT(3);
 	FunnelPlan rplan;
 	st = mx == kBad32 ? kResidualReconciliationMagnitudeOutOfDomain : funnel_plan(mx, &ss, 1, a.res_site, &rplan);
@@ -2619,14 +2633,12 @@ __global__ __launch_bounds__(BS) void k_residual_norm(sslm_launch::ResidualArgs 
 	KT(4);
 	int8_t* out = a.out_stream + (size_t)oidx * H;
 	int32_t c[EPT];
+	const double rfac = requant_factor(rplan.r, rplan.s);
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) {
 		const int i = threadIdx.x + k * BS;
-		c[k] = 0;
-		if (i < H) {
-			c[k] = requant_code_f(w[k], requant_factor(rplan.r, rplan.s));
-			out[i] = (int8_t)c[k];
-		}
+		c[k] = requant_code_d(w[k], rfac);  // 0 past H
+		if (i < H) out[i] = (int8_t)c[k];
 	}
 	if (threadIdx.x == 0) a.out_stream_scale[oidx] = rplan.out;
 	KT(5);
@@ -5042,6 +5054,7 @@ void funnel(const FunnelArgs& a, hipStream_t s) {
 }
 
 void residual_norm(const ResidualArgs& a, hipStream_t s) {
+	if (a.raw.part && a.raw.epi.seg[0].bias) throw LaunchRefused{"residual_norm: a projection with a bias"};
 	// decode launches (a few rows, one block each on otherwise idle CUs) of long rows: 1024
 	// threads per row, so each thread's share of the row and of its raw planes is half as long
 	// (measured: 7B rows of 3584 gain, 1.5B rows of 1536 at 3 per thread lose)
