@@ -20,20 +20,19 @@ compile() {
   grep -v "packed-fp32-ops" "$log" >&2 || true
   rm -f "$log"
 }
-compile csrc/kernels.hip _build/kernels.o &
-P1=$!
-compile csrc/runtime.cpp _build/runtime.o &
-P2=$!
-compile csrc/artifact.cpp _build/artifact.o &
-P3=$!
-compile csrc/noalloc.hip _build/noalloc.o &
-P4=$!
+PIDS=()
+OBJS=()
+for src in csrc/*.hip csrc/*.cpp; do
+  obj=_build/$(basename "${src%.*}").o
+  OBJS+=("$obj")
+  compile "$src" "$obj" &
+  PIDS+=($!)
+done
 FAIL=0
-for p in $P1 $P2 $P3 $P4; do wait $p || FAIL=1; done
+for p in "${PIDS[@]}"; do wait "$p" || FAIL=1; done
 if [ $FAIL -ne 0 ]; then
   rm -f libsslm_hip.so
   exit 1
 fi
-hipcc -shared -fPIC --offload-arch=gfx950 _build/kernels.o _build/runtime.o _build/artifact.o \
-  _build/noalloc.o -lcrypto -o libsslm_hip.so.tmp
+hipcc -shared -fPIC --offload-arch=gfx950 "${OBJS[@]}" -lcrypto -o libsslm_hip.so.tmp
 mv libsslm_hip.so.tmp libsslm_hip.so

@@ -721,6 +721,34 @@ SSLM_HD double norm_qd(int32_t v, double root, double inv) {
 	const double r = fma(-q, root, n);
 	return r < 0.0 ? q - 1.0 : (r >= root ? q + 1.0 : q);
 }
+// 1 / d to within 2^-40 of itself, for quotient estimates that an exact remainder corrects: on the GPU
+// the hardware reciprocal and one Newton step instead of the division sequence
+SSLM_HD double rcp_est(double d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+	const double r = __builtin_amdgcn_rcp(d);
+	return fma(r, fma(-d, r, 1.0), r);
+#else
+	return 1.0 / d;
+#endif
+}
+
+// The RMSNorm's root (forward_sites.cpp:410-459): isqrt(floor(ss 2^32 / h)), at least 1, for a row
+// of h <= 2^13 codes with sum of squares ss <= 2^14 h.  floor(sqrt(floor(x))) = floor(sqrt(x)), so it is
+// the largest r with r^2 h <= ss 2^32 (r <= 2^23, every product below 2^61): a double estimate of
+// sqrt(ss 2^32 / h), within 2^-15 of it, and one exact step each way.
+SSLM_HD int64_t rms_root(int32_t ss, int32_t h) {
+	const uint64_t n = (uint64_t)(uint32_t)ss << 32, uh = (uint64_t)(uint32_t)h;
+	const double x = (double)(ss > 0 ? ss : 1) * 4294967296.0 * rcp_est((double)h);
+#if defined(__HIP_DEVICE_COMPILE__)
+	const double y = __builtin_amdgcn_rsq(x), r0 = x * y;
+	uint32_t r = (uint32_t)fma(0.5 * y, fma(-r0, r0, x), r0);  // one Newton step from 2^-22
+#else
+	uint32_t r = (uint32_t)sqrt(x);
+#endif
+	r -= (uint64_t)r * r * uh > n ? 1u : 0u;
+	r += ((uint64_t)r + 1) * ((uint64_t)r + 1) * uh <= n ? 1u : 0u;
+	return ss > 0 && r > 1 ? r : 1;
+}
 SSLM_HD int64_t norm_fd(int32_t v, double root, double inv) { return (int64_t)norm_qd(v, root, inv); }
 
 SSLM_HD int64_t softmax_ceiling(int64_t q_b, int64_t q_c) {

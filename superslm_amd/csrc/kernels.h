@@ -135,6 +135,7 @@ struct LaunchRefused {
 };
 
 void gemm(const GemmArgs& g, hipStream_t s);
+int device_cus();  // compute units of the current device
 // launch shape of the decode GEMV (M <= 64, K % 128 == 0); `split_ok`: the caller consumes raw
 // split-K partials; `raw_or_argmax`: no projection epilogue in the kernel (raw accumulators or
 // argmax keys)
@@ -364,6 +365,21 @@ void mlp_act(const ActArgs& a, hipStream_t s);
 // M <= kMaxSlicedActRows.
 bool mlp_act_sliced_ok(const ActArgs& a);
 void mlp_act_sliced(const ActArgs& a, hipStream_t s);
+void mlp_act_products(const ActArgs& a, hipStream_t s);  // its first launch alone (products, maxima, scales)
+int act_slices(int I);                                   // the slices it writes maxima of
+
+// ---- decode of a few sequences: each funnel inside the GEMV that reads its codes (decode_chain.hip) ----
+constexpr int kChainRows = 4;
+// whether funnel_gemv and act_gemv, and at M = 1 residual_gemv, take a layer of this geometry (no LoRA,
+// packed weights)
+bool decode_chain_ok(int M, int H, int NH, int KVH, int I);
+// funnel() then gemm() of its codes (raw output)
+void funnel_gemv(const GemmArgs& g, const FunnelArgs& a, hipStream_t s);
+// residual_norm() of one row on a raw projection, then gemm() of its norm's codes (g.epi's bias
+// reconcile takes the norm's own scales)
+void residual_gemv(const GemmArgs& g, const ResidualArgs& a, hipStream_t s);
+// the second launch of mlp_act_sliced(), then gemm() of its codes (split-K planes)
+void act_gemv(const GemmArgs& g, const ActArgs& a, hipStream_t s);
 
 // whether the row kernels' register tiling covers this geometry
 bool row_geometry_ok(int H, int I, int NKV, int D);

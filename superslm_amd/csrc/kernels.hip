@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstdlib>
 
+#include "device_util.h"
 #include "kernels.h"
 
 // Optional phase timestamps for latency studies of the row kernels; compiled out by default.
@@ -18,10 +19,6 @@
 #endif
 
 namespace sslm {
-
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v2i __attribute__((ext_vector_type(2)));
-typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kBlock = 256;
 constexpr int kRowBlock = 1024;  // row kernels: one block per token
@@ -62,28 +59,11 @@ __device__ __forceinline__ uint64_t block_max_u64(uint64_t v, uint64_t* red) {
 	return r;
 }
 
-// Row maxima travel as 32-bit magnitudes: |v| saturated at 2^32 - 2, so that 2^32 - 1 (kBad32)
-// is free to mark a refusal somewhere in the row.  Every consumer rejects a maximum above 2^31
-// (the funnel's accepted domain), so the saturation changes no outcome.
-constexpr uint32_t kBad32 = 0xffffffffu;
-
-__device__ __forceinline__ uint32_t sat_abs_u32(int64_t v) {
-	uint64_t a = v < 0 ? (uint64_t)0 - (uint64_t)v : (uint64_t)v;
-	return a > 0xfffffffeull ? 0xfffffffeu : (uint32_t)a;
-}
-
-// sat_abs_u32 of a row maximum held in a non-negative double
-__device__ __forceinline__ uint32_t sat_u32_d(double m) { return (uint32_t)fmin(m, 4294967294.0); }
-
 // The row of a one-block-per-row launch: workgroups go to the 8 XCDs in turn (block b on XCD
 // b % 8), so giving each XCD a contiguous run of rows keeps a tile-major maxima array's lines
 // ([tile][row], 32 rows to a line) in one XCD's L2 instead of fetched by all eight.  Identity
 // when the row count is not a multiple of 8.
 __device__ __forceinline__ int xcd_row(int b, int n) { return (n & 7) ? b : (b & 7) * (n >> 3) + (b >> 3); }
-
-__device__ __forceinline__ int32_t sat_i32(int64_t v) {
-	return v > kI32Max ? kI32Max : (v < kI32Min ? kI32Min : (int32_t)v);
-}
 
 // ------------------------------------------------------------------------------------------
 // projection epilogue: WSC1 fold -> LoRA delta -> bias reconcile (forward_sites.cpp:1114-1141)
@@ -174,8 +154,6 @@ __device__ __forceinline__ void epi_store(const Epilogue& e, const EpiResult& r,
 	}
 }
 
-__device__ __forceinline__ v4i load16(const int8_t* p) { return *(const v4i*)p; }
-
 // One output element (token t, channel j) of any GEMM: raw accumulator, argmax key, or the
 // projection epilogue; returns the element's contribution to its tile's partial max.
 __device__ __forceinline__ void epi_element(const Epilogue& e, int N, int t, int j, int32_t acc, uint64_t* key,
@@ -228,42 +206,12 @@ __device__ __forceinline__ void epi_publish(const Epilogue& e, int tile, int t, 
 // epilogue; with several, each split stores its raw partial plane and the consumer adds them
 // (no cross-block synchronisation inside the kernel).
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t dpp_max16(uint32_t v) {
-	// row_ror:8, 4, 2, 1 -- every lane of the 16-lane row ends with the row maximum
-	uint32_t w = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false);
-	v = w > v ? w : v;
-	w = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false);
-	v = w > v ? w : v;
-	w = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, false);
-	v = w > v ? w : v;
-	w = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false);
-	return w > v ? w : v;
-}
-
 // Refused bias reconciles in the decode GEMV epilogue (rare; out of line): bit v of `mask` marks
 // token t0 + v.
 __device__ __attribute__((noinline)) void set_status_rows(int32_t* status, const TokenInfo* tok, int32_t layer, int t0,
                                                          uint32_t mask) {
 	for (int v = 0; v < 4; ++v)
 		if (mask >> v & 1) set_status(status, tok[t0 + v].slot, layer, kBiasReconcileProductOutOfDomain);
-}
-
-// The fields of segment `si` (wave-uniform) that the decode GEMV epilogue uses, selected with
-// constant indices so they stay scalar kernel-argument loads.
-struct SegView {
-	int32_t n_begin, mode, ld_out;
-	void* out;
-	uint32_t* maxpart;
-	const int32_t* fold;
-	const int64_t* bias;
-	const int8_t* lora_b;
-	const int32_t* lora_dfold;
-	const int8_t* lora_u;
-};
-
-__device__ __forceinline__ SegView seg_view(const Epilogue& e, int si) {
-	const Segment& s = si == 0 ? e.seg[0] : (si == 1 ? e.seg[1] : e.seg[2]);
-	return SegView{s.n_begin, s.mode, s.ld_out, s.out, s.maxpart, s.fold, s.bias, s.lora_b, s.lora_dfold, s.lora_u};
 }
 
 constexpr int kGemvWaves = 4;
@@ -452,12 +400,6 @@ __global__ __launch_bounds__(64 * kGemvWaves) void k_gemv(GemmArgs g, int cps) {
 // reduce -> epilogue runs once per block with nothing behind it: gate|up at 16 tokens with
 // HBM-cold weights 11.5 -> 9 us.
 // ------------------------------------------------------------------------------------------
-// segment of the 16-column tile starting at column c0 (bounds are multiples of 16), with
-// constant indices so the fields stay scalar kernel-argument loads
-__device__ __forceinline__ int tile_segment(const Epilogue& e, int c0) {
-	return (e.nseg > 1 && c0 >= e.seg[0].n_end) ? ((e.nseg > 2 && c0 >= e.seg[1].n_end) ? 2 : 1) : 0;
-}
-
 template <int MB, int CPW>  // MB row groups of 16 tokens
 __global__ __launch_bounds__(256) void k_gemv_p(GemmArgs g) {
 	__shared__ v4i red[2][kGemvWaves][MB][64];
@@ -561,8 +503,6 @@ __global__ __launch_bounds__(256) void k_gemv_p(GemmArgs g) {
 // as INT32_MIN).  Each block reads the activation rows once for all its tiles, where one block
 // per tile pair read them once per 32 columns.
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ const int8_t* pk_lane(const int8_t* wp, int tile, int C, int lane);
-
 constexpr int kHeadMaxSteps = 64;  // tiles per block of k_gemv_head (the launch sizes its grid to fit)
 
 // Four row groups (M 33..64) over more than 16 chunks take eight waves of CPW chunks (NW = 8, as in
@@ -693,11 +633,6 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_head(GemmArgs g) {
 // column l % 16).  Measured against k_gemv on the 1.5B decode shapes with every layer's weights
 // streaming from HBM: LM head 59 -> 49 us, down projection (8 planes) 8.4 -> 6.4 us.
 // ------------------------------------------------------------------------------------------
-// lane `lane`'s 16 bytes of chunk 0, half 0 of `tile` in a packed decode copy (k_gemv_pk)
-__device__ __forceinline__ const int8_t* pk_lane(const int8_t* wp, int tile, int C, int lane) {
-	return wp + (size_t)tile * C * 2048 + lane * 16;
-}
-
 // PK: the weights are read from the packed decode copy g.wp (see k_gemv_pk), the activations
 // with its lane -> k map.
 template <int NCH, bool PK>
@@ -1922,33 +1857,6 @@ __global__ __launch_bounds__(kRowBlock) void k_embed(const int32_t* tokens, cons
 // A slot's status is read once by thread 0 and tested after the first barrier, so the whole
 // block leaves together.
 // ------------------------------------------------------------------------------------------
-// A block reduction's result is the same in every lane; saying so (readfirstlane) lets the
-// compiler keep it, and the scalar scale plans computed from it, in scalar registers.
-__device__ __forceinline__ uint64_t uni_u64(uint64_t v) {
-	const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-	const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-	return ((uint64_t)hi << 32) | lo;
-}
-__device__ __forceinline__ int64_t uni_i64(int64_t v) { return (int64_t)uni_u64((uint64_t)v); }
-
-// 32-bit wave reductions: a 16-lane rotate butterfly (DPP) leaves every lane with its row's
-// result, and the four row results are read as scalars -- the value comes back wave-uniform.
-__device__ __forceinline__ uint32_t wave_max32(uint32_t v) {
-	v = dpp_max16(v);
-	const uint32_t a = __builtin_amdgcn_readlane(v, 0), b = __builtin_amdgcn_readlane(v, 16);
-	const uint32_t c = __builtin_amdgcn_readlane(v, 32), d = __builtin_amdgcn_readlane(v, 48);
-	return max(max(a, b), max(c, d));
-}
-
-__device__ __forceinline__ int32_t wave_sum32(int32_t v) {
-	v += __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, false);  // row_ror:8
-	v += __builtin_amdgcn_update_dpp(0, v, 0x124, 0xf, 0xf, false);  // row_ror:4
-	v += __builtin_amdgcn_update_dpp(0, v, 0x122, 0xf, 0xf, false);  // row_ror:2
-	v += __builtin_amdgcn_update_dpp(0, v, 0x121, 0xf, 0xf, false);  // row_ror:1
-	return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16) + __builtin_amdgcn_readlane(v, 32) +
-	       __builtin_amdgcn_readlane(v, 48);
-}
-
 // block reductions with one barrier; each call site owns its LDS slots (BS / 64 entries)
 template <int BS>
 __device__ __forceinline__ uint32_t blk_max32(uint32_t v, uint32_t* slots) {
@@ -2120,10 +2028,8 @@ __device__ __forceinline__ int32_t rmsnorm_regs(const int32_t (&h)[EPT], const i
 	ss = blk_sum32<BS>(ss, s_sum);
 	KT(10);
 	if (prior && *prior != 0) return kSkipped;
-	int64_t root = isqrt_fast(div_floor_pos((int64_t)ss << 32, (int64_t)H));
-	root = root > 1 ? root : 1;
-	// floor((v << 32) / root) per element from one shared reciprocal (root < 2^23)
-	const double rd = (double)root, inv = 1.0 / rd;
+	// floor((v << 32) / root) per element from one shared reciprocal estimate (root <= 2^23)
+	const double rd = (double)rms_root(ss, H), inv = rcp_est(rd);
 	KT(11);
 	double w[EPT], mxd = 0.0;  // |quotient * gain| < 2^39 * 2^7: exact in doubles
 #pragma unroll
@@ -4343,8 +4249,6 @@ static bool gemv_persistent_ok(const GemmArgs& g) {
 	return true;
 }
 
-static int device_cus();
-
 template <int MB>
 void launch_gemv_p(const GemmArgs& g, hipStream_t s) {
 	const int C = g.K >> 7, T = (g.N + 15) / 16;
@@ -4362,7 +4266,7 @@ void launch_gemv_p(const GemmArgs& g, hipStream_t s) {
 }
 
 // compute units of the current device (one persistent block each)
-static int device_cus() {
+int device_cus() {
 	static const int n = [] {
 		int dev = 0, cus = 0;
 		if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
@@ -5105,21 +5009,30 @@ bool mlp_act_sliced_ok(const ActArgs& a) {
 	       a.I <= kMaxActSlices * kActSliceMax;
 }
 
-void mlp_act_sliced(const ActArgs& a, hipStream_t s) {
-	const int S = std::max(1, std::min(kMaxActSlices, (a.I + kActSliceMax - 1) / kActSliceMax));
-	const int per = ((a.I + S - 1) / S + 15) / 16 * 16;
-	const int ept = (per + kActSliceBS - 1) / kActSliceBS;
-	const dim3 grid(a.M, (a.I + per - 1) / per);
+// columns per slice of a row of I
+static int act_slice_cols(int I) {
+	const int S = std::max(1, std::min(kMaxActSlices, (I + kActSliceMax - 1) / kActSliceMax));
+	return ((I + S - 1) / S + 15) / 16 * 16;
+}
+
+int act_slices(int I) { return (I + act_slice_cols(I) - 1) / act_slice_cols(I); }
+
+static void launch_act_slices(const ActArgs& a, bool codes, hipStream_t s) {
+	const int per = act_slice_cols(a.I), ept = (per + kActSliceBS - 1) / kActSliceBS;
+	const dim3 grid(a.M, act_slices(a.I));
 #define X(E)                                                                                                  \
 	if (ept <= E) {                                                                                           \
 		hipLaunchKernelGGL((k_mlp_act_s1<kActSliceBS, E>), grid, dim3(kActSliceBS), 0, s, a, per);             \
-		hipLaunchKernelGGL((k_mlp_act_s2<kActSliceBS, E>), grid, dim3(kActSliceBS), 0, s, a, per);             \
+		if (codes) hipLaunchKernelGGL((k_mlp_act_s2<kActSliceBS, E>), grid, dim3(kActSliceBS), 0, s, a, per);  \
 		return;                                                                                               \
 	}
 	X(1) X(2) X(3) X(4) X(5)
 #undef X
 	no_instance("mlp_act_sliced", a.I);
 }
+
+void mlp_act_sliced(const ActArgs& a, hipStream_t s) { launch_act_slices(a, true, s); }
+void mlp_act_products(const ActArgs& a, hipStream_t s) { launch_act_slices(a, false, s); }
 
 bool row_geometry_ok(int H, int I, int NKV, int D) {
 	return H <= 16 * kRowBS && H <= 16 * kFunnelBS && I <= 20 * kActBS && NKV * D <= 4 * kRowBS && H / 2 <= 8 * kRowBS &&

@@ -571,12 +571,18 @@ Segment funnel_seg(int n0, int n1, int32_t* out, int ld, uint32_t* mx, const int
 	return s;
 }
 
-void run_gemm(sslm_model m, Track& w, const GemmArgs& g, int cls) {
+// `launch` enqueues the GEMM g, or a kernel that holds it.
+template <typename F>
+void run_gemm_as(Track& w, const GemmArgs& g, int cls, F&& launch) {
 	const int64_t out_bytes = g.epi.argmax_key ? 0 : (int64_t)g.M * g.N * 4;
 	ProfScope p(w.stream, cls, (int64_t)g.N * g.K + (int64_t)g.M * g.K + 12LL * g.N + out_bytes,
 	            2LL * g.M * g.N * g.K, profile_shape_key(cls, g.M, g.N, g.K));
-	sslm_launch::gemm(g, w.stream);
+	launch();
 	ck(hipGetLastError());
+}
+
+void run_gemm(sslm_model m, Track& w, const GemmArgs& g, int cls) {
+	run_gemm_as(w, g, cls, [&] { sslm_launch::gemm(g, w.stream); });
 }
 
 // Decode projections (and prefill GEMMs that split K) hand their raw partial planes to the next
@@ -828,12 +834,18 @@ void run_layers(sslm_model m, Track& w, int M, StreamRef st, int l0, int l1, ssl
 	const bool fused = decode && M <= kTrackTokens && H % 128 == 0 && fused_attention_enabled();
 	const bool staged_attn = !decode && w.kv_stage && sslm_launch::tiled_attention_staged(M, m->NKV, m->NH);
 	const bool dbg = dbg_on(m, M);
+	// a few sequences: the context and activation funnels run inside the GEMVs that read their codes, for
+	// one sequence the residual rows too (the q|k|v projection of layers past the first in the one before)
+	const DevLayer& lp = m->layers[l0];
+	const bool chain = fused && !ad && !dbg && w.raw_part && lp.p_qkv && lp.p_o && lp.p_gu && lp.p_down && w.act_prod &&
+	                   sslm_launch::decode_chain_ok(M, H, m->NH, KVH, I);
+	const bool chain_rows = chain && M == 1;
 	for (int l = l0; l < l1; ++l) {
 		const DevLayer& lw = m->layers[l];
 		RawIn raw{};  // the last projection's split-K partials, when it split
 		if (dbg) dbg_gather(m, w, l, kDbgAttnNorm, w.normed, w.normed_scale, nullptr, H, M);
 		// q | k | v projection (forward_sites.cpp:1699-1735)
-		{
+		if (!chain_rows || l == l0) {
 			const int pj[3] = {0, 1, 2};
 			run_lora_u(m, w, ad, l, pj, 3, w.normed, M, H);
 			ProjArgs pa = qkv_args(m, w, l, M, ad, fused);
@@ -929,12 +941,18 @@ void run_layers(sslm_model m, Track& w, int M, StreamRef st, int l0, int l1, ssl
 			a.layer = l;
 			a.status = m->status;
 			a.head_status = m->head_status;
-			ProfScope p(s, kProfRow, 0, 0);
-			sslm_launch::funnel(a, s);
-			ck(hipGetLastError());
+			if (chain) {
+				ProjArgs pa = o_args(m, w, l, M, nullptr);
+				raw = pa.raw;
+				run_gemm_as(w, pa.g, kProfGemm, [&] { sslm_launch::funnel_gemv(pa.g, a, s); });
+			} else {
+				ProfScope p(s, kProfRow, 0, 0);
+				sslm_launch::funnel(a, s);
+				ck(hipGetLastError());
+			}
 			if (dbg) dbg_gather(m, w, l, kDbgCtx, w.ctx, w.ctx_scale, nullptr, H, M);
 		}
-		{  // o_proj (forward_sites.cpp:1907-1914)
+		if (!chain) {  // o_proj (forward_sites.cpp:1907-1914)
 			const int pj[1] = {3};
 			run_lora_u(m, w, ad, l, pj, 1, w.ctx, M, H);
 			ProjArgs pa = o_args(m, w, l, M, ad);
@@ -966,15 +984,21 @@ void run_layers(sslm_model m, Track& w, int M, StreamRef st, int l0, int l1, ssl
 			a.status = m->status;
 			a.raw = raw;
 			if (dbg) a.branch_tap = dbg_tap(m, l, kDbgO);
-			ProfScope p(s, kProfRow, 0, 0);
-			sslm_launch::residual_norm(a, s);
-			ck(hipGetLastError());
+			if (chain_rows) {  // with the gate | up projection
+				const GemmArgs gu = gu_args(m, w, l, M, nullptr).g;
+				run_gemm_as(w, gu, kProfGemm, [&] { sslm_launch::residual_gemv(gu, a, s); });
+				raw = RawIn{};
+			} else {
+				ProfScope p(s, kProfRow, 0, 0);
+				sslm_launch::residual_norm(a, s);
+				ck(hipGetLastError());
+			}
 			if (dbg) {
 				dbg_gather(m, w, l, kDbgAttnRes, w.attn_stream, w.attn_stream_scale, nullptr, H, M);
 				dbg_gather(m, w, l, kDbgMlpNorm, w.mlp_normed, w.mlp_scale, nullptr, H, M);
 			}
 		}
-		{  // gate | up (forward_sites.cpp:1938-1955)
+		if (!chain_rows) {  // gate | up (forward_sites.cpp:1938-1955)
 			const int pj[2] = {4, 5};
 			run_lora_u(m, w, ad, l, pj, 2, w.mlp_normed, M, H);
 			ProjArgs pa = gu_args(m, w, l, M, ad);
@@ -1005,15 +1029,26 @@ void run_layers(sslm_model m, Track& w, int M, StreamRef st, int l0, int l1, ssl
 				a.gate_tap = dbg_tap(m, l, kDbgGate);
 				a.up_tap = dbg_tap(m, l, kDbgUp);
 			}
-			ProfScope p(s, kProfRow, 0, 0);
-			// short launches: one block per (row, column slice) in two launches, instead of one
-			// block per row that leaves most CUs idle (see kSlicedActPrefillRows)
-			if ((decode || M <= kSlicedActPrefillRows) && sslm_launch::mlp_act_sliced_ok(a)) sslm_launch::mlp_act_sliced(a, s);
-			else sslm_launch::mlp_act(a, s);
-			ck(hipGetLastError());
-			if (dbg) dbg_gather(m, w, l, kDbgAct, w.act, w.act_scale, nullptr, I, M);
+			if (chain) {  // the products, then the activation funnel with the down projection
+				{
+					ProfScope p(s, kProfRow, 0, 0);
+					sslm_launch::mlp_act_products(a, s);
+					ck(hipGetLastError());
+				}
+				ProjArgs pa = down_args(m, w, l, M, nullptr);
+				raw = pa.raw;
+				run_gemm_as(w, pa.g, kProfGemm, [&] { sslm_launch::act_gemv(pa.g, a, s); });
+			} else {
+				ProfScope p(s, kProfRow, 0, 0);
+				// short launches: one block per (row, column slice) in two launches, instead of one
+				// block per row that leaves most CUs idle (see kSlicedActPrefillRows)
+				if ((decode || M <= kSlicedActPrefillRows) && sslm_launch::mlp_act_sliced_ok(a)) sslm_launch::mlp_act_sliced(a, s);
+				else sslm_launch::mlp_act(a, s);
+				ck(hipGetLastError());
+				if (dbg) dbg_gather(m, w, l, kDbgAct, w.act, w.act_scale, nullptr, I, M);
+			}
 		}
-		{  // down_proj (forward_sites.cpp:1969-1977)
+		if (!chain) {  // down_proj (forward_sites.cpp:1969-1977)
 			const int pj[1] = {6};
 			run_lora_u(m, w, ad, l, pj, 1, w.act, M, I);
 			ProjArgs pa = down_args(m, w, l, M, ad);
@@ -1047,9 +1082,14 @@ void run_layers(sslm_model m, Track& w, int M, StreamRef st, int l0, int l1, ssl
 			a.status = m->status;
 			a.raw = raw;
 			if (dbg) a.branch_tap = dbg_tap(m, l, kDbgDown);
-			ProfScope p(s, kProfRow, 0, 0);
-			sslm_launch::residual_norm(a, s);
-			ck(hipGetLastError());
+			if (chain_rows && a.gain) {  // with the next layer's q | k | v projection
+				const GemmArgs qkv = qkv_args(m, w, l + 1, M, nullptr, true).g;
+				run_gemm_as(w, qkv, kProfGemm, [&] { sslm_launch::residual_gemv(qkv, a, s); });
+			} else {
+				ProfScope p(s, kProfRow, 0, 0);
+				sslm_launch::residual_norm(a, s);
+				ck(hipGetLastError());
+			}
 			if (dbg) dbg_gather(m, w, l, kDbgMlpRes, st.codes, st.scale, st.idx, H, M);
 		}
 	}

@@ -73,6 +73,13 @@ int main(int argc, char** argv) {
 			const int64_t n = r * r + d;
 			if (n >= 0) EXPECT(isqrt_fast(n) == or_isqrt(n), "%lld", (long long)n);
 		}
+	// the RMSNorm's root
+	for (long i = 0; i < N; ++i) {
+		const int32_t h = (int32_t)(i % 3 ? uni(1, 8192) : 64 * uni(1, 128));
+		const int32_t ss = (int32_t)(i % 5 ? uni(0, 16384LL * h) : uni(0, 4096));
+		const int64_t want = or_isqrt(((int64_t)ss << 32) / h);
+		EXPECT(rms_root(ss, h) == (want > 1 ? want : 1), "rms_root %d / %d", ss, h);
+	}
 	// requant code on the funnel's domain
 	for (long i = 0; i < N; ++i) {
 		const int64_t x = uni(-(1LL << 31), 1LL << 31);
