@@ -516,6 +516,34 @@ SSLM_HD int64_t landing_small(int64_t branch, int64_t m_a, int64_t r_t, int64_t 
 
 SSLM_HD int64_t clamp_code(int64_t v) { return v > 127 ? 127 : (v < -127 ? -127 : v); }
 
+// The landed code of a K or V value, clamp_code(landing_rescale(...)), and its clamp flag, from a
+// double estimate.  p = |m_a| r_t and f = p 2^-k are common to a head, so a value is one product:
+// x = |branch| f is within 200 * 2^-50 of the exact magnitude below 200, and rounding it half up is exact
+// unless x + 1/2 lies within 1e-9 of an integer.  That band, a product past 2^126 or a quotient past
+// 2^62 (where the 128-bit form wraps) take the exact form out of line: inlined at each value
+// it was most of its kernels' instruction bytes, which a launch fetches cold.
+struct LandingScale {
+	double p, f;
+};
+SSLM_HD LandingScale landing_scale(int64_t m_a, int64_t r_t, int64_t k) {
+	const uint64_t am = m_a < 0 ? (uint64_t)0 - (uint64_t)m_a : (uint64_t)m_a;
+	LandingScale s;
+	s.p = (double)am * (double)(uint64_t)r_t;
+	s.f = ldexp(s.p, (int)-k);
+	return s;
+}
+SSLM_HD int32_t landing_code(int64_t branch, int64_t m_a, int64_t r_t, int64_t k, const LandingScale& s, bool* clamped) {
+	const double ab = fabs((double)branch), x = ab * s.f, y = x + 0.5, q = floor(y), d = y - q;
+	if (!(ab * s.p < 0x1p126) || !(x < 0x1p62) || (x < 200.0 && (d < 1e-9 || d > 1.0 - 1e-9))) {
+		const Landing l = landing_rescale_cold(branch, m_a, r_t, k);
+		*clamped = l.clamped;
+		return (int32_t)clamp_code(l.raw);
+	}
+	*clamped = q > 127.0;
+	const int32_t c = (int32_t)fmin(q, 127.0);
+	return (branch < 0) != (m_a < 0) ? -c : c;
+}
+
 // forward_sites.cpp:399-408
 SSLM_HD int64_t floor_div(int64_t a, int64_t b) {
 	int64_t q = a / b, r = a % b;
@@ -629,6 +657,8 @@ SSLM_HD int64_t div_rcp(int64_t n, int64_t d, double inv, int64_t qmax) {
 	return q;
 }
 
+SSLM_COLD int64_t div_rcp_cold(int64_t n, int64_t d, double inv, int64_t qmax) { return div_rcp(n, d, inv, qmax); }
+
 // iexp_element (intmath.cpp:580-668) for a row whose constants passed check_softmax_width
 // (q_c >= 0, q_b^2 + q_c <= kSoftmaxMaxSafe) and shifted <= 0:
 // the quotient z in [0, 30] from a reciprocal, and the square in 64 bits when |base| < 2^31
@@ -655,6 +685,11 @@ SSLM_HD int64_t iexp_fast(int64_t shifted, int64_t q_ln2, double inv_ln2, int64_
 	else value = (int64_t)((((s128)base * base) + (s128)q_c) >> z);
 	if (m_ceiling <= 0 || value < 0 || value > m_ceiling) return -1;
 	return value;
+}
+
+// out of line, for kernels whose rows almost always admit iexp_small (code size)
+SSLM_COLD int64_t iexp_fast_cold(int64_t shifted, int64_t q_ln2, double inv_ln2, int64_t q_b, int64_t q_c, int64_t m_ceiling) {
+	return iexp_fast(shifted, q_ln2, inv_ln2, q_b, q_c, m_ceiling);
 }
 
 // The softmax's per-element ceiling M = q_b^2 + q_c when usable (intmath.cpp:831-851), else 0.

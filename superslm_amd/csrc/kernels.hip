@@ -2075,9 +2075,13 @@ __global__ __launch_bounds__(BS) void k_rmsnorm(sslm_launch::RowNormArgs a, int 
 }
 
 // q funnel + RoPE(q); K/V landing, RoPE(K), KV write (forward_sites.cpp:1281-1418, :1748-1787).
-// The K/V landing does not depend on the q funnel, so it is computed while the q maximum is
-// reduced.  Up to 2 K (and 2 V) pairs per thread: NKV * D <= 4 * BS.
-template <int BS, int EQ, int RS>
+// Latency-bound, one block per token.  The row's pairs -- q, then K, then V, in the projection's column
+// order -- are spread evenly over the threads (NP each), every load is issued before the first
+// use, and the K/V landing, which does not depend on the q funnel, is computed while the q maximum is
+// reduced.  A launch fetches its instructions cold, so one landing body serves K and V
+// (128-bit landings inlined at each of eight values, 24 KB of code: 9.4-10.1 us at hidden 1536, now
+// 12 KB and 6.6-7.1; past a thousand rows of hidden 3584 the spare slots cost, 27 -> 33 us of 2 ms a layer).
+template <int BS, int NP, int RS>
 __global__ __launch_bounds__(BS) void k_qkv_post(sslm_launch::QkvPostArgs a) {
 	__shared__ uint32_t s_red[BS / 64];
 	__shared__ int32_t s_st;
@@ -2085,90 +2089,140 @@ __global__ __launch_bounds__(BS) void k_qkv_post(sslm_launch::QkvPostArgs a) {
 	const TokenInfo ti = a.tok[t];
 	const Scale ns = a.in_scale[t];
 	const int H = a.H, D = a.D, pairs = D / 2;
-	const int KVH = a.NKV * D;
+	const int KVH = a.NKV * D, Q = H / 2, KP = KVH / 2, P = Q + KVH;  // pairs: q, K (and V), all
 	const int64_t pos = ti.pos;
 	const bool pos_ok = pos >= 0 && pos < a.cap;
 	const int64_t* cs = a.rope_cos + (pos_ok ? pos : 0) * pairs;
 	const int64_t* sn = a.rope_sin + (pos_ok ? pos : 0) * pairs;
-	// q pair values
-	int2 qv[EQ];
-	uint32_t qmx = 0;
-	if (RS > 0) {
-		int j[2 * EQ];
-		bool live[2 * EQ];
-		int64_t v[2 * EQ];
+	const float rpairs = 1.0f / (float)pairs;
+	int pi[NP], hd[NP];  // pair within its head, KV head (q pairs: the first)
+	int64_t v0[NP], v1[NP], rt[NP], et[NP];
+	int32_t cc[NP], sc[NP];
+#define SSLM_PAIR(k)                                       \
+	const int p = min((int)threadIdx.x + k * BS, P - 1);     \
+	const bool live = (int)threadIdx.x + k * BS < P;         \
+	const bool isq = p < Q, isk = !isq && p < Q + KP;        \
+	const int kvi = isq ? 0 : p - (isk ? Q : Q + KP); /* K or V pair */
 #pragma unroll
-		for (int k = 0; k < EQ; ++k) {
-			const int p = threadIdx.x + k * BS;
-			j[2 * k] = 2 * p;
-			j[2 * k + 1] = 2 * p + 1;
-			live[2 * k] = live[2 * k + 1] = p < H / 2;
+	for (int k = 0; k < NP; ++k) {
+		SSLM_PAIR(k)
+		(void)live;
+		const int hh = (int)(((float)p + 0.5f) * rpairs);  // p / pairs: half a pair from the next integer, p < 2^13
+		pi[k] = p - hh * pairs;
+		hd[k] = isq ? 0 : hh - (isk ? a.NH : a.NH + a.NKV);
+		(void)kvi;
+		rt[k] = et[k] = 0;
+		cc[k] = sc[k] = 0;
+		if (!isq) {  // (whole waves, but for a boundary's)
+			rt[k] = (isk ? a.r_t_k : a.r_t_v)[hd[k]];
+			et[k] = (isk ? a.e_t_k : a.e_t_v)[hd[k]];
 		}
-		const bool ok = raw_row<2 * EQ, RS>(a.raw, 0, a.M, t, j, live, v);
+		if (isq || isk) {
+			cc[k] = (int32_t)cs[pi[k]];
+			sc[k] = (int32_t)sn[pi[k]];
+		}
+	}
+	uint32_t qmx = 0;
+	const int32_t status0 = a.status[ti.slot];
+	if constexpr (RS > 0) {
+		// the raw planes' two columns with their folds and biases (raw_row's rules; the accumulators,
+		// below 2^29, admit the bounded fold)
+		const Epilogue& e = a.raw.epi;
+		const size_t plane = (size_t)a.M * a.raw.ld;
+		const int32_t* row = a.raw.part + (size_t)t * a.raw.ld;
+		int2 acc[NP];
+		int32_t f[NP][6];
+		int64_t b0[NP], b1[NP];
+		const bool any_bias = e.seg[0].bias || e.seg[1].bias || e.seg[2].bias;
+		const int64_t rcp = any_bias ? e.in_recip[t] : 0, ein = any_bias ? e.in_scale[t].e : 0;
 #pragma unroll
-		for (int k = 0; k < EQ; ++k) {
-			qv[k] = make_int2(sat_i32(v[2 * k]), sat_i32(v[2 * k + 1]));
-			qmx = max(qmx, max(sat_abs_u32(v[2 * k]), sat_abs_u32(v[2 * k + 1])));
+		for (int k = 0; k < NP; ++k) {
+			SSLM_PAIR(k)
+			(void)live;
+			uint32_t s0 = 0, s1 = 0;
+#pragma unroll
+			for (int s2 = 0; s2 < RS; ++s2) {  // clamped plane index: no branch, no extra round trip
+				const int2 x = *(const int2*)(row + (size_t)(RS == 1 ? 0 : min(s2, a.raw.splits - 1)) * plane + 2 * p);
+				s0 += RS == 1 || s2 < a.raw.splits ? (uint32_t)x.x : 0u;  // the true sum fits int32; partials wrap harmlessly
+				s1 += RS == 1 || s2 < a.raw.splits ? (uint32_t)x.y : 0u;
+			}
+			acc[k] = make_int2((int)s0, (int)s1);
+			const int jj = isq ? 2 * p : 2 * kvi;
+			const int32_t* fp = (isq ? e.seg[0].fold : (isk ? e.seg[1].fold : e.seg[2].fold)) + 3 * jj;
+#pragma unroll
+			for (int i = 0; i < 6; ++i) f[k][i] = fp[i];
+			const int64_t* bp = isq ? e.seg[0].bias : (isk ? e.seg[1].bias : e.seg[2].bias);
+			b0[k] = bp ? bp[jj] : 0;
+			b1[k] = bp ? bp[jj + 1] : 0;
+		}
+		bool ok = true;
+#pragma unroll
+		for (int k = 0; k < NP; ++k) {
+			SSLM_PAIR(k)
+			v0[k] = fold_bounded(acc[k].x, fold_consts(f[k][0], f[k][1], f[k][2]));
+			v1[k] = fold_bounded(acc[k].y, fold_consts(f[k][3], f[k][4], f[k][5]));
+			const int8_t* lb = isq ? e.seg[0].lora_b : (isk ? e.seg[1].lora_b : e.seg[2].lora_b);
+			if (lb) {
+				const int8_t* lu = isq ? e.seg[0].lora_u : (isk ? e.seg[1].lora_u : e.seg[2].lora_u);
+				const int32_t* df = isq ? e.seg[0].lora_dfold : (isk ? e.seg[1].lora_dfold : e.seg[2].lora_dfold);
+				const int jj = isq ? 2 * p : 2 * kvi;
+				v0[k] += lora_delta_cold(lb, lu, df, e.rank, t, jj);
+				v1[k] += lora_delta_cold(lb, lu, df, e.rank, t, jj + 1);
+			}
+			if (isq ? e.seg[0].bias != nullptr : (isk ? e.seg[1].bias != nullptr : e.seg[2].bias != nullptr)) {
+				int64_t t0 = 0, t1 = 0;
+				const bool o = bias_term(b0[k], rcp, ein, v0[k], &t0) & bias_term(b1[k], rcp, ein, v1[k], &t1);
+				v0[k] += t0;
+				v1[k] += t1;
+				if (live && !o) ok = false;
+			}
+			if (live && isq) qmx = max(qmx, max(sat_abs_u32(v0[k]), sat_abs_u32(v1[k])));
 		}
 		if (!ok) qmx = kBad32;
 	} else {
 		const int2* qf = (const int2*)(a.q_f + (size_t)t * H);
-		int2 qr[EQ];
+		const longlong2* kv = (const longlong2*)(a.kv_f + (size_t)t * 2 * KVH);
+		int2 qr[NP];
+		longlong2 kr[NP];
 #pragma unroll
-		for (int k = 0; k < EQ; ++k) qr[k] = qf[min((int)threadIdx.x + k * BS, H / 2 - 1)];  // clamped: no per-lane branch
-#pragma unroll
-		for (int k = 0; k < EQ; ++k) qv[k] = (int)threadIdx.x + k * BS < H / 2 ? qr[k] : make_int2(0, 0);
-		qmx = part_max32_fixed<BS, (2 * EQ + 15) / 16>(a.q_maxpart, 0, H / 16, t);  // H <= 2 * EQ * BS
-	}
-	if (threadIdx.x == 0) s_st = a.status[ti.slot];
-	// K/V landing (LandingRescale at the normed scale, per kv head) and RoPE(K)
-	const int64_t* kv = RS > 0 ? nullptr : a.kv_f + (size_t)t * 2 * KVH;
-	int8_t kq[2][2], vq[2][2];
-	uint64_t sat = 0;
-	int64_t rk[4], rv[4];
-	if (RS > 0) {
-		int jk[4], jv[4];
-		bool live[4];
-#pragma unroll
-		for (int k = 0; k < 2; ++k) {
-			const int p = threadIdx.x + k * BS;
-			jk[2 * k] = H + 2 * p;
-			jk[2 * k + 1] = H + 2 * p + 1;
-			jv[2 * k] = H + KVH + 2 * p;
-			jv[2 * k + 1] = H + KVH + 2 * p + 1;
-			live[2 * k] = live[2 * k + 1] = p < KVH / 2;
+		for (int k = 0; k < NP; ++k) {
+			const int p = min((int)threadIdx.x + k * BS, P - 1);
+			qr[k] = make_int2(0, 0);
+			kr[k] = make_longlong2(0, 0);
+			if (p < Q) qr[k] = qf[p];
+			else kr[k] = kv[p - Q];
 		}
-		const bool okk = raw_row<4, RS>(a.raw, 1, a.M, t, jk, live, rk);
-		const bool okv = raw_row<4, RS>(a.raw, 2, a.M, t, jv, live, rv);
-		if (!(okk && okv)) qmx = kBad32;
-	}
+		qmx = part_max32_fixed<BS, (2 * NP + 15) / 16>(a.q_maxpart, 0, H / 16, t);  // H <= 2 NP BS
 #pragma unroll
-	for (int k = 0; k < 2; ++k) {
-		const int p = threadIdx.x + k * BS;
-		if (p < KVH / 2) {  // (an out-of-range position is refused below; its values are unused)
-			const int hd = (2 * p) / D;
-			const int i = p % pairs;
-			longlong2 kk, vv;
-			if (RS > 0) {
-				kk = make_longlong2(rk[2 * k], rk[2 * k + 1]);
-				vv = make_longlong2(rv[2 * k], rv[2 * k + 1]);
-			} else {
-				kk = ((const longlong2*)kv)[p];
-				vv = ((const longlong2*)(kv + KVH))[p];
+		for (int k = 0; k < NP; ++k) {
+			const bool isq = (int)threadIdx.x + k * BS < Q;
+			v0[k] = isq ? (int64_t)qr[k].x : (int64_t)kr[k].x;
+			v1[k] = isq ? (int64_t)qr[k].y : (int64_t)kr[k].y;
+		}
+	}
+	if (threadIdx.x == 0) s_st = status0;
+	// K/V landing (LandingRescale at the normed scale, per kv head) and RoPE(K); an out-of-range position is
+	// refused below, its values are unused
+	char2 kvc[NP];
+	uint32_t sat = 0;
+#pragma unroll
+	for (int k = 0; k < NP; ++k) {
+		SSLM_PAIR(k)
+		(void)kvi;
+		kvc[k] = make_char2(0, 0);
+		if (live && !isq) {
+			const int64_t ke = composed_exponent(ns.e, et[k]);
+			const LandingScale ls = landing_scale(ns.m, rt[k], ke);
+			bool c0, c1;
+			const int32_t x = landing_code(v0[k], ns.m, rt[k], ke, ls, &c0);
+			const int32_t y = landing_code(v1[k], ns.m, rt[k], ke, ls, &c1);
+			sat += (uint32_t)c0 + (uint32_t)c1;
+			kvc[k] = make_char2((char)x, (char)y);
+			if (isk) {
+				int64_t xr, yr;
+				rope_pair(x, y, cc[k], sc[k], &xr, &yr);
+				kvc[k] = make_char2((char)clamp_code(xr), (char)clamp_code(yr));
 			}
-			const int64_t k_e = composed_exponent(ns.e, a.e_t_k[hd]);
-			const int64_t v_e = composed_exponent(ns.e, a.e_t_v[hd]);
-			const int64_t rtk = a.r_t_k[hd], rtv = a.r_t_v[hd];
-			bool c0, c1, c2, c3, x0;
-			const int64_t k0 = clamp_code(landing_rescale(kk.x, ns.m, rtk, k_e, &c0, &x0));
-			const int64_t k1 = clamp_code(landing_rescale(kk.y, ns.m, rtk, k_e, &c1, &x0));
-			int64_t xr, yr;
-			rope_pair((int32_t)k0, (int32_t)k1, (int32_t)cs[i], (int32_t)sn[i], &xr, &yr);
-			kq[k][0] = (int8_t)clamp_code(xr);
-			kq[k][1] = (int8_t)clamp_code(yr);
-			vq[k][0] = (int8_t)clamp_code(landing_rescale(vv.x, ns.m, rtv, v_e, &c2, &x0));
-			vq[k][1] = (int8_t)clamp_code(landing_rescale(vv.y, ns.m, rtv, v_e, &c3, &x0));
-			sat += (uint64_t)c0 + (uint64_t)c1 + (uint64_t)c2 + (uint64_t)c3;
 		}
 	}
 	qmx = blk_max32<BS>(qmx, s_red);
@@ -2180,52 +2234,38 @@ __global__ __launch_bounds__(BS) void k_qkv_post(sslm_launch::QkvPostArgs a) {
 		if (threadIdx.x == 0) set_status(a.status, ti.slot, a.layer, st);
 		return;
 	}
-	// q: codes of pair (2i, 2i+1), rotated, clamped
+	// q: codes of pair (2i, 2i+1), rotated, clamped; K/V: to the staging row (prefill spans: until every
+	// token's q funnel has passed) or the pool
+	const double qfac = requant_factor(plan.r, plan.s);
 	char2* qo = (char2*)(a.q_rot + (size_t)t * H);
-#pragma unroll
-	for (int k = 0; k < EQ; ++k) {
-		const int p = threadIdx.x + k * BS;
-		if (p < H / 2) {
-			const int i = p % pairs;
-			const int32_t x = requant_code_f(qv[k].x, requant_factor(plan.r, plan.s));
-			const int32_t y = requant_code_f(qv[k].y, requant_factor(plan.r, plan.s));
-			int64_t xr, yr;
-			rope_pair(x, y, (int32_t)cs[i], (int32_t)sn[i], &xr, &yr);
-			qo[p] = make_char2((char)clamp_code(xr), (char)clamp_code(yr));
-		}
-	}
-	if (threadIdx.x == 0) a.q_scale[t] = plan.out;
-	if (a.kv_stage) {  // prefill span: staged until every token's q funnel has passed
-		int8_t* row = a.kv_stage + (size_t)t * 2 * KVH;
-#pragma unroll
-		for (int k = 0; k < 2; ++k) {
-			const int p = threadIdx.x + k * BS;
-			if (p < KVH / 2) {
-				*(char2*)(row + 2 * p) = make_char2(kq[k][0], kq[k][1]);
-				*(char2*)(row + KVH + 2 * p) = make_char2(vq[k][0], vq[k][1]);
-			}
-		}
-		sat = wave_sum_i64((int64_t)sat);
-		if ((threadIdx.x & 63) == 0 && sat) atomicAdd(&a.sat_stage[t], (uint32_t)sat);
-		return;
-	}
+	int8_t* stage = a.kv_stage ? a.kv_stage + (size_t)t * 2 * KVH : nullptr;
 	int8_t* blk = a.kv_pool + (int64_t)ti.block * a.block_bytes;
 	const int64_t half = a.cap * (int64_t)KVH;
-	int8_t* kstore = blk + (int64_t)a.layer * half * 2;
-	int8_t* vstore = kstore + half;
 #pragma unroll
-	for (int k = 0; k < 2; ++k) {
-		const int p = threadIdx.x + k * BS;
-		if (p < KVH / 2) {
-			const int hd = (2 * p) / D;
-			const int i = p % pairs;
-			const int64_t off = ((int64_t)hd * a.cap + pos) * D + 2 * i;
-			*(char2*)(kstore + off) = make_char2(kq[k][0], kq[k][1]);
-			*(char2*)(vstore + off) = make_char2(vq[k][0], vq[k][1]);
+	for (int k = 0; k < NP; ++k) {
+		SSLM_PAIR(k)
+		if (!live) continue;
+		if (isq) {
+			int64_t xr, yr;
+			// (RS = 0: the funnel's own 32-bit values)
+			const int32_t q0 = RS > 0 ? sat_i32(v0[k]) : (int32_t)v0[k], q1 = RS > 0 ? sat_i32(v1[k]) : (int32_t)v1[k];
+			rope_pair(requant_code_f(q0, qfac), requant_code_f(q1, qfac), cc[k], sc[k], &xr, &yr);
+			qo[p] = make_char2((char)clamp_code(xr), (char)clamp_code(yr));
+		} else if (stage) {
+			*(char2*)(stage + 2 * (p - Q)) = kvc[k];
+		} else {
+			int8_t* dst = blk + (int64_t)a.layer * half * 2 + (isk ? 0 : half);
+			*(char2*)(dst + ((int64_t)hd[k] * a.cap + pos) * D + 2 * pi[k]) = kvc[k];
 		}
+		(void)kvi;
 	}
-	sat = wave_sum_i64((int64_t)sat);
-	if ((threadIdx.x & 63) == 0 && sat) atomicAdd(&a.sat[ti.slot], (unsigned long long)sat);
+#undef SSLM_PAIR
+	if (threadIdx.x == 0) a.q_scale[t] = plan.out;
+	const int32_t ws = wave_sum32((int32_t)sat);
+	if ((threadIdx.x & 63) == 0 && ws) {
+		if (stage) atomicAdd(&a.sat_stage[t], (uint32_t)ws);
+		else atomicAdd(&a.sat[ti.slot], (unsigned long long)ws);
+	}
 }
 
 // Looped form of k_slot_state_copy for rows or K/V spans past its fixed per-thread counts.
@@ -2937,20 +2977,30 @@ __global__ __launch_bounds__(BS) void k_attention(sslm_launch::AttnArgs a) {
 		if (s_st != 0) return;
 		uint32_t sat = 0;
 		char2 kc = make_char2(0, 0), vc = make_char2(0, 0);
-		if (kthr) {  // the K landing and RoPE(K) of pair ic
-			bool c0, c1, x0;
-			const int64_t k0 = clamp_code(landing_rescale(kk.x, ns.m, rtk, k_e, &c0, &x0));
-			const int64_t k1 = clamp_code(landing_rescale(kk.y, ns.m, rtk, k_e, &c1, &x0));
-			int64_t xr, yr;
-			rope_pair((int32_t)k0, (int32_t)k1, c, sn, &xr, &yr);
-			kc = make_char2((char)clamp_code(xr), (char)clamp_code(yr));
+		if (kthr || vthr) {  // the landing of pair ic: K, rotated, and / or V
+			bool c0, c1;
+			const bool kf = kthr;  // the K pair (threads with both: the V pair after it)
+			const int64_t rt = kf ? rtk : rtv, ex2 = kf ? k_e : v_e;
+			const LandingScale ls = landing_scale(ns.m, rt, ex2);
+			const int32_t x = landing_code(kf ? kk.x : vv.x, ns.m, rt, ex2, ls, &c0);
+			const int32_t y = landing_code(kf ? kk.y : vv.y, ns.m, rt, ex2, ls, &c1);
 			sat += (uint32_t)c0 + (uint32_t)c1;
-			((char2*)s_kc)[ic] = kc;
+			if (kf) {
+				int64_t xr, yr;
+				rope_pair(x, y, c, sn, &xr, &yr);
+				kc = make_char2((char)clamp_code(xr), (char)clamp_code(yr));
+				((char2*)s_kc)[ic] = kc;
+			} else {
+				vc = make_char2((char)x, (char)y);
+				((char2*)s_vc)[ic] = vc;
+			}
 		}
-		if (vthr) {  // the V landing of pair ic
-			bool c2, c3, x0;
-			vc = make_char2((char)clamp_code(landing_rescale(vv.x, ns.m, rtv, v_e, &c2, &x0)),
-			                (char)clamp_code(landing_rescale(vv.y, ns.m, rtv, v_e, &c3, &x0)));
+		if (!SPLITV && vthr) {
+			bool c2, c3;
+			const LandingScale ls = landing_scale(ns.m, rtv, v_e);
+			const int32_t x = landing_code(vv.x, ns.m, rtv, v_e, ls, &c2);
+			const int32_t y = landing_code(vv.y, ns.m, rtv, v_e, ls, &c3);
+			vc = make_char2((char)x, (char)y);
 			sat += (uint32_t)c2 + (uint32_t)c3;
 			((char2*)s_vc)[ic] = vc;
 		}
@@ -3196,6 +3246,8 @@ __global__ __launch_bounds__(BS) void k_attention(sslm_launch::AttnArgs a) {
 // scores through the passes: a span of at most 128 positions reads K once (100 prompts of 4-12
 // tokens and their decoding 293.6 -> 280.4 ms).  4-wave blocks, held to 3 a CU, have no registers
 // for either (2,048-token 7B attention 321 -> 369 us with them): k_kv_commit runs before them.
+// The general i-exp and quotient of rows past the 32-bit forms are called out of line: inlined eight
+// times they were 10 KB of the kernel, fetched cold by each launch (4-12 tokens 12.7 -> 11.8 us).
 constexpr int kTiledECache = 512;  // positions whose i-exp values an 8-wave tiled-attention block keeps
 
 template <int D, int NW>
@@ -3388,7 +3440,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 	}
 	auto iexp_tok = [&](int v, int64_t shifted) {
 		return esmall[v] ? iexp_small(shifted, (int32_t)cq[v][0], inv[v], (int32_t)cq[v][1], cq[v][2], cq[v][3])
-		                 : iexp_fast(shifted, cq[v][0], inv[v], cq[v][1], cq[v][2], cq[v][3]);
+		                 : iexp_fast_cold(shifted, cq[v][0], inv[v], cq[v][1], cq[v][2], cq[v][3]);
 	};
 	__syncthreads();
 	// pass 2: i-exp values (SoftmaxRowQ15, intmath.cpp:853-889) and the row sums
@@ -3464,7 +3516,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 				// e <= total, so the quotient is at most 2^15
 				const int64_t e = ecache ? s_e[NW == 8 ? g * 4 + v : 0][NW == 8 ? p : 0] : iexp_tok(v, (int64_t)s[v] - rmx[v]);
 				pr = e == 0 ? 0
-				            : (dsmall[v] ? div_q15_small(e, ddn[v], dinv[v]) : (int32_t)div_rcp(e << 15, denom[v], dinv[v], 32768));
+				            : (dsmall[v] ? div_q15_small(e, ddn[v], dinv[v]) : (int32_t)div_rcp_cold(e << 15, denom[v], dinv[v], 32768));
 			}
 			s_p[0][g * 4 + v][pl] = (int8_t)(pr >> 14);
 			s_p[1][g * 4 + v][pl] = (int8_t)((pr >> 7) & 127);
@@ -3656,20 +3708,29 @@ __global__ __launch_bounds__(64 * NW, 1) void k_attention_group(sslm_launch::Att
 	// what another writes)
 	uint32_t sat = 0;
 	char2 kc = make_char2(0, 0), vc = make_char2(0, 0);
-	if (kthr) {
-		bool c0, c1, x0;
-		const int64_t k0 = clamp_code(landing_rescale(kk.x, ns.m, rtk, k_e, &c0, &x0));
-		const int64_t k1 = clamp_code(landing_rescale(kk.y, ns.m, rtk, k_e, &c1, &x0));
-		int64_t xr, yr;
-		rope_pair((int32_t)k0, (int32_t)k1, ck, sk, &xr, &yr);
-		kc = make_char2((char)clamp_code(xr), (char)clamp_code(yr));
+	if (kthr || vthr) {  // K, rotated, or V
+		bool c0, c1;
+		const int64_t rt = kthr ? rtk : rtv, ex2 = kthr ? k_e : v_e;
+		const LandingScale ls = landing_scale(ns.m, rt, ex2);
+		const int32_t x = landing_code(kthr ? kk.x : vv.x, ns.m, rt, ex2, ls, &c0);
+		const int32_t y = landing_code(kthr ? kk.y : vv.y, ns.m, rt, ex2, ls, &c1);
 		sat += (uint32_t)c0 + (uint32_t)c1;
-		((char2*)s_kc)[ki] = kc;
+		if (kthr) {
+			int64_t xr, yr;
+			rope_pair(x, y, ck, sk, &xr, &yr);
+			kc = make_char2((char)clamp_code(xr), (char)clamp_code(yr));
+			((char2*)s_kc)[ki] = kc;
+		} else {
+			vc = make_char2((char)x, (char)y);
+			((char2*)s_vc)[ki] = vc;
+		}
 	}
-	if (vthr) {
-		bool c2, c3, x0;
-		vc = make_char2((char)clamp_code(landing_rescale(vv.x, ns.m, rtv, v_e, &c2, &x0)),
-		                (char)clamp_code(landing_rescale(vv.y, ns.m, rtv, v_e, &c3, &x0)));
+	if (!splitv && vthr) {  // short of threads: V after K
+		bool c2, c3;
+		const LandingScale ls = landing_scale(ns.m, rtv, v_e);
+		const int32_t x = landing_code(vv.x, ns.m, rtv, v_e, ls, &c2);
+		const int32_t y = landing_code(vv.y, ns.m, rtv, v_e, ls, &c3);
+		vc = make_char2((char)x, (char)y);
 		sat += (uint32_t)c2 + (uint32_t)c3;
 		((char2*)s_vc)[ki] = vc;
 	}
@@ -4742,7 +4803,7 @@ void rmsnorm(const RowNormArgs& a, int M, int H, const TokenInfo* tok, int32_t* 
 }
 
 void qkv_post(const QkvPostArgs& a, hipStream_t s) {
-	const int need = row_ept(a.H / 2, kRowBS);
+	const int need = row_ept(a.H / 2 + a.NKV * a.D, kRowBS);
 #define X(E)                                                                                          \
 	if (need <= E) {                                                                                  \
 		if (!a.raw.part) hipLaunchKernelGGL((k_qkv_post<kRowBS, E, 0>), dim3(a.M), dim3(kRowBS), 0, s, a); \
@@ -4750,7 +4811,7 @@ void qkv_post(const QkvPostArgs& a, hipStream_t s) {
 		else hipLaunchKernelGGL((k_qkv_post<kRowBS, E, kMaxRawSplits>), dim3(a.M), dim3(kRowBS), 0, s, a); \
 		return;                                                                                       \
 	}
-	X(1) X(2) X(4) X(8)
+	X(1) X(2) X(3) X(5) X(8) X(12)  // at most 8 of q (H / 2 <= 8 kRowBS) and 4 of K and V
 #undef X
 	no_instance("qkv_post", a.H);
 }

@@ -132,6 +132,31 @@ int main(int argc, char** argv) {
 			EXPECT(requant_code_f(x, requant_factor(r, s)) == or_requant_code_wide(x, r, s), "tie %lld %d", (long long)x, s);
 			EXPECT(or_requant_code_wide(x, r, s) == (sg ? -64 : 64), "tie rounds away from zero");
 		}
+	// landed K/V codes by double estimate: every exponent band, values at and beside half-integers, and
+	// operands whose product or quotient passes the estimate's domain
+	for (long i = 0; i < N * 4; ++i) {
+		const int vb = (int)uni(1, i % 16 ? 34 : 63);
+		int64_t v = (int64_t)(rng() >> (64 - vb)) * (rng() & 1 ? 1 : -1);
+		int64_t m_a = uni(1LL << 30, (1LL << 31) - 1) * (rng() % 8 ? 1 : -1);
+		int64_t r_t = i % 32 ? uni(1LL << 31, 1LL << 32) : (int64_t)(rng() >> uni(0, 40));
+		int64_t k = uni(40, 110);
+		if (i % 4 == 0) {  // |v| m_a r_t / 2^k = n + 1/2, or one off in v
+			m_a = 1LL << 30;
+			r_t = 1LL << 32;
+			const int s = (int)uni(0, 20);
+			k = 62 + 1 + s;
+			v = (2 * uni(0, 140) + 1) * (1LL << s) + uni(-1, 1);
+			if (rng() & 1) v = -v;
+		}
+		if (i % 64 == 7) k = uni(-200, 200);
+		if (i % 64 == 9) v = 0;
+		if (i % 256 == 11) k = rng() & 1 ? 4096 : -4096;
+		bool cl1, cl2, ex2;
+		const int32_t got = landing_code(v, m_a, r_t, k, landing_scale(m_a, r_t, k), &cl1);
+		const int64_t want = clamp_code(landing_rescale(v, m_a, r_t, k, &cl2, &ex2));
+		EXPECT(got == want && cl1 == cl2, "%lld %lld %lld %lld: %d %lld", (long long)v, (long long)m_a, (long long)r_t, (long long)k,
+		       got, (long long)want);
+	}
 	// landing on residual operands, every exponent band
 	for (long i = 0; i < N; ++i) {
 		const int64_t branch = uni(-127, 127);
