@@ -41,6 +41,21 @@ __device__ __forceinline__ uint32_t dpp_max16(uint32_t v) {
 	return w > v ? w : v;
 }
 
+// maximum / sum over each 16-lane row, in every lane of it
+__device__ __forceinline__ int32_t row16_max(int32_t v) { return (int32_t)(dpp_max16((uint32_t)v ^ 0x80000000u) ^ 0x80000000u); }
+template <int CTRL>
+__device__ __forceinline__ int64_t row16_rot(int64_t v) {
+	const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, 0xf, 0xf, false);
+	const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)((uint64_t)v >> 32), CTRL, 0xf, 0xf, false);
+	return (int64_t)((uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ int64_t row16_sum(int64_t v) {
+	v += row16_rot<0x128>(v);
+	v += row16_rot<0x124>(v);
+	v += row16_rot<0x122>(v);
+	return v + row16_rot<0x121>(v);
+}
+
 // The fields of segment `si` (wave-uniform) that the decode GEMV epilogue uses, selected with
 // constant indices so they stay scalar kernel-argument loads.
 struct SegView {

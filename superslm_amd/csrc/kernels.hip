@@ -3248,6 +3248,11 @@ __global__ __launch_bounds__(BS) void k_attention(sslm_launch::AttnArgs a) {
 // for either (2,048-token 7B attention 321 -> 369 us with them): k_kv_commit runs before them.
 // The general i-exp and quotient of rows past the 32-bit forms are called out of line: inlined eight
 // times they were 10 KB of the kernel, fetched cold by each launch (4-12 tokens 12.7 -> 11.8 us).
+// A short tile is one chain of dependent phases, so nothing waits that need not: the last wave derives
+// the i-exp constants (4,000 cycles of 25,000) while the others run pass 1, the committed rows are
+// loaded at entry with the operands (the round trip was 3,200), rows reduce by DPP rotations instead of
+// LDS permutes, and the four tokens' i-exp chains interleave where all admit the 32-bit form
+// (4-12 tokens 11.8 -> 10.5 us, 512 tokens 31.9 -> 28.3, 2,048 of 7B 323 -> 314).
 constexpr int kTiledECache = 512;  // positions whose i-exp values an 8-wave tiled-attention block keeps
 
 template <int D, int NW>
@@ -3318,10 +3323,17 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 		qa[c] = ri < nt && off_ok ? qa[c] : v4i{0, 0, 0, 0};
 		if (STAGED) k0r[c] = off_ok ? k0r[c] : v4i{0, 0, 0, 0};
 	}
+	// this thread's 16 bytes of the tile's K/V rows for the pool, in the blocks that commit them
+	const bool commit = STAGED && h % group == 0;
+	const int ctq = threadIdx.x / (D / 8), ckv = threadIdx.x % (D / 8) / (D / 16), cch = threadIdx.x % (D / 16);
+	static_assert(NW != 8 || TQ * (D / 8) <= 64 * NW, "a chunk per thread");
+	v4i crow = v4i{0, 0, 0, 0};
+	if (commit && ctq < nt) crow = load16(kstage + (int64_t)ckv * KVH + (int64_t)(t0 + ctq) * (2 * KVH) + cch * 16);
 	if (threadIdx.x == 0) s_st = st0;
-	if (threadIdx.x < TQ) {
-		// the token's i-exp constants and width, as k_attention derives them
-		const int tq = threadIdx.x;
+	// The last wave derives the tokens' i-exp constants and widths, as k_attention does; the others go
+	// on to pass 1, which needs neither.
+	if (threadIdx.x >= 64 * (NW - 1) && lane < TQ) {
+		const int tq = lane;
 		int32_t st = kOk;
 		int64_t c0 = 0, c1 = 0, c2 = 0, cm = 0, pos = -1;
 		if (tq < nt) {
@@ -3354,36 +3366,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 		s_mab[tq] = 0;
 		s_rf[tq] = 0;
 	}
-	__syncthreads();
-	if (STAGED && h == 0 && threadIdx.x < nt) {  // the tile's clamp counts, cleared whatever the status
-		const uint32_t sat = a.sat_stage[t0 + threadIdx.x];
-		a.sat_stage[t0 + threadIdx.x] = 0;
-		if (s_st == 0 && sat) atomicAdd(&a.sat[ti0.slot], (unsigned long long)sat);
-	}
-	if (s_st != 0) return;
-	if (STAGED && h % group == 0) {  // the tile's K/V rows of this KV head, into the pool
-		for (int c = threadIdx.x; c < nt * (D / 8); c += 64 * NW) {
-			const int tq = c / (D / 8), r = c % (D / 8), kv = r / (D / 16), ch = r % (D / 16);
-			int8_t* dst = (int8_t*)(kv ? vbase : kbase) + (int64_t)(span0 + t0 + tq) * D + ch * 16;
-			*(v4i*)dst = load16(kstage + (int64_t)kv * KVH + (int64_t)(t0 + tq) * (2 * KVH) + ch * 16);
-		}
-	}
-	if (threadIdx.x < nt && s_ok[threadIdx.x] != kOk)
-		report_head(a.head_status, ti0.slot, h, s_ok[threadIdx.x] == -1 ? kPositionOverCap : s_ok[threadIdx.x]);
-	int wmax = 0;  // positions [0, wmax) cover every live token's row
-	for (int tq = 0; tq < nt; ++tq)
-		if (s_ok[tq] == kOk) wmax = max(wmax, s_pos[tq] + 1);
-	if (wmax == 0) return;
-	// the output tokens of this lane: g*4 + v
-	int32_t tpos[4];
-	bool tok_ok[4];
-#pragma unroll
-	for (int v = 0; v < 4; ++v) {
-		tpos[v] = s_pos[g * 4 + v];
-		tok_ok[v] = s_ok[g * 4 + v] == kOk;
-	}
-	const int nblk = (wmax + KB - 1) / KB;
-	const bool ecache = NW == 8 && nblk * KB <= ECP;
+	// positions [0, wtile) cover the tile's rows within the cap; the output tokens of this lane are
+	// g*4 + v, at positions tp0 + v (past nt: dropped by tok_ok)
+	const int wtile = (int)max((int64_t)0, min(ti0.pos + nt, a.cap));
+	const int32_t tp0 = (int32_t)ti0.pos + g * 4;
 	auto scores = [&](int blk, int* p_out) {
 		const int p = blk * KB + wave * 16 + ri;
 		const int8_t* kr = k_row(p);
@@ -3406,20 +3392,38 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 	int32_t mx[4] = {INT32_MIN, INT32_MIN, INT32_MIN, INT32_MIN};
 #pragma unroll
 	for (int v = 0; v < 4; ++v)
-		if (STAGED && tok_ok[v] && p0 <= tpos[v]) mx[v] = s0[v];
-	for (int blk = STAGED ? 1 : 0; blk < nblk; ++blk) {
+		if (STAGED && p0 <= tp0 + v) mx[v] = s0[v];
+	for (int blk = STAGED ? 1 : 0; blk * KB < wtile; ++blk) {
 		int p;
 		const v4i s = scores(blk, &p);
 #pragma unroll
 		for (int v = 0; v < 4; ++v)
-			if (tok_ok[v] && p <= tpos[v]) mx[v] = max(mx[v], s[v]);
+			if (p <= tp0 + v) mx[v] = max(mx[v], s[v]);
 	}
 #pragma unroll
 	for (int v = 0; v < 4; ++v) {
-		for (int o = 8; o > 0; o >>= 1) mx[v] = max(mx[v], __shfl_xor(mx[v], o, 16));
+		mx[v] = row16_max(mx[v]);
 		if (ri == 0) s_red[wave][g * 4 + v] = mx[v];
 	}
 	__syncthreads();
+	if (STAGED && h == 0 && threadIdx.x < nt) {  // the tile's clamp counts, cleared whatever the status
+		const uint32_t sat = a.sat_stage[t0 + threadIdx.x];
+		a.sat_stage[t0 + threadIdx.x] = 0;
+		if (s_st == 0 && sat) atomicAdd(&a.sat[ti0.slot], (unsigned long long)sat);
+	}
+	if (s_st != 0) return;
+	if (commit && ctq < nt)  // the tile's K/V rows of this KV head, into the pool
+		*(v4i*)((int8_t*)(ckv ? vbase : kbase) + (int64_t)(span0 + t0 + ctq) * D + cch * 16) = crow;
+	if (threadIdx.x < nt && s_ok[threadIdx.x] != kOk)
+		report_head(a.head_status, ti0.slot, h, s_ok[threadIdx.x] == -1 ? kPositionOverCap : s_ok[threadIdx.x]);
+	// positions [0, wmax) cover every live token's row
+	const int wmax = __builtin_amdgcn_readfirstlane(row16_max(s_ok[ri] == kOk ? s_pos[ri] + 1 : 0));
+	if (wmax == 0) return;
+	bool tok_ok[4];
+#pragma unroll
+	for (int v = 0; v < 4; ++v) tok_ok[v] = s_ok[g * 4 + v] == kOk;
+	const int nblk = (wmax + KB - 1) / KB;
+	const bool ecache = NW == 8 && nblk * KB <= ECP;
 	int64_t rmx[4];
 #pragma unroll
 	for (int v = 0; v < 4; ++v) {
@@ -3436,8 +3440,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 #pragma unroll
 		for (int i = 0; i < 4; ++i) cq[v][i] = s_c[g * 4 + v][i];
 		inv[v] = s_inv[g * 4 + v];
-		esmall[v] = iexp_small_ok(cq[v][0], cq[v][1], cq[v][3]);
+		esmall[v] = !tok_ok[v] || iexp_small_ok(cq[v][0], cq[v][1], cq[v][3]);  // (a dead row's values are dropped)
 	}
+	const bool all_small = __all(esmall[0] && esmall[1] && esmall[2] && esmall[3]);
 	auto iexp_tok = [&](int v, int64_t shifted) {
 		return esmall[v] ? iexp_small(shifted, (int32_t)cq[v][0], inv[v], (int32_t)cq[v][1], cq[v][2], cq[v][3])
 		                 : iexp_fast_cold(shifted, cq[v][0], inv[v], cq[v][1], cq[v][2], cq[v][3]);
@@ -3450,9 +3455,20 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 		int p = p0;
 		v4i s = s0;
 		if (!STAGED || blk > 0) s = scores(blk, &p);
+		if (NW == 8 && all_small) {  // the four tokens' chains interleave
+#pragma unroll
+			for (int v = 0; v < 4; ++v) {
+				const bool in = tok_ok[v] && p <= tp0 + v;
+				const int64_t e = iexp_small((int64_t)s[v] - rmx[v], (int32_t)cq[v][0], inv[v], (int32_t)cq[v][1], cq[v][2], cq[v][3]);
+				if (ecache && in) s_e[NW == 8 ? g * 4 + v : 0][NW == 8 ? p : 0] = e;
+				refused |= in && e < 0 ? 1u << v : 0u;
+				sum[v] += in && e >= 0 ? e : 0;
+			}
+			continue;
+		}
 #pragma unroll
 		for (int v = 0; v < 4; ++v) {
-			if (tok_ok[v] && p <= tpos[v]) {
+			if (tok_ok[v] && p <= tp0 + v) {
 				const int64_t e = iexp_tok(v, (int64_t)s[v] - rmx[v]);
 				if (ecache) s_e[NW == 8 ? g * 4 + v : 0][NW == 8 ? p : 0] = e;
 				if (e < 0) refused |= 1u << v;
@@ -3462,11 +3478,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 	}
 #pragma unroll
 	for (int v = 0; v < 4; ++v) {
-		for (int o = 8; o > 0; o >>= 1) sum[v] += __shfl_xor(sum[v], o, 16);
+		sum[v] = row16_sum(sum[v]);
 		if (ri == 0) s_red[wave][g * 4 + v] = sum[v];
 	}
-	for (int o = 8; o > 0; o >>= 1) refused |= __shfl_xor(refused, o, 16);
-	if (ri == 0 && refused)
+	if (refused)
 		for (int v = 0; v < 4; ++v)
 			if (refused >> v & 1) s_rf[g * 4 + v] = 1;
 	__syncthreads();
@@ -3512,7 +3527,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void k_attention_tiled(ss
 #pragma unroll
 		for (int v = 0; v < 4; ++v) {
 			int32_t pr = 0;
-			if (tok_ok[v] && p <= tpos[v]) {
+			if (tok_ok[v] && p <= tp0 + v) {
 				// e <= total, so the quotient is at most 2^15
 				const int64_t e = ecache ? s_e[NW == 8 ? g * 4 + v : 0][NW == 8 ? p : 0] : iexp_tok(v, (int64_t)s[v] - rmx[v]);
 				pr = e == 0 ? 0
