@@ -86,7 +86,6 @@ __global__ __launch_bounds__(512) void k_residual_gemv(GemmArgs g, sslm_launch::
 	constexpr int PD = NI * CPW <= 12 ? NI : (NI < 2 ? NI : 2);
 	__shared__ __attribute__((aligned(16))) int8_t s_x[1][LDX];
 	__shared__ int32_t red[NI][NW][16];
-	__shared__ double land[256];
 	__shared__ uint32_t s_m[3][NW];
 	__shared__ int32_t s_s[NW];
 	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -174,23 +173,17 @@ __global__ __launch_bounds__(512) void k_residual_gemv(GemmArgs g, sslm_launch::
 		if (lead && rl == 0) set_status(a.status, slot, a.layer, st);
 		ok = false;
 	}
-	// ---- residual: the landed value of each branch code, tabulated ----
-	if (rl < 256) {
-		const int64_t r_h = reciprocal_fast(ok ? ss.m : ((int64_t)1 << 30));
-		const int64_t kx = composed_exponent(bp.out.e, ss.e);
-		bool cl, ex;
-		const int64_t rec = landing_small((int64_t)min(rl, 254) - 127, bp.out.m, r_h, kx, &cl, &ex);
-		land[rl] = ex ? (double)INFINITY : (double)rec;
-	}
-	const double bf = requant_factor(bp.r, bp.s);
+	// ---- residual: the landed value of each branch code ----
+	const int64_t r_h = reciprocal_fast(ok ? ss.m : ((int64_t)1 << 30)), kx = composed_exponent(bp.out.e, ss.e);
+	const double lf = landing_scale(bp.out.m, r_h, kx).f;
+	const double bf = bp.f;
 	int32_t c[EP];
 #pragma unroll
 	for (int k = 0; k < EP; ++k) c[k] = ok ? requant_code_f(bv[k], bf) : 0;
-	__syncthreads();
 	double w[EP], mxd = 0.0;
 #pragma unroll
 	for (int k = 0; k < EP; ++k) {
-		w[k] = rl + k * RT < H ? land[c[k] + 127] + (double)sv[k] : 0.0;
+		w[k] = rl + k * RT < H ? residual_land(c[k], bp.out.m, r_h, kx, lf) + (double)sv[k] : 0.0;
 		mxd = fmax(mxd, fabs(w[k]));
 	}
 	mx = row_max<NW>(mxd == (double)INFINITY ? kBad32 : sat_u32_d(mxd), s_m[1]);
@@ -199,7 +192,7 @@ __global__ __launch_bounds__(512) void k_residual_gemv(GemmArgs g, sslm_launch::
 		if (lead && rl == 0) set_status(a.status, slot, a.layer, st);
 		ok = false;
 	}
-	const double rf = requant_factor(rp.r, rp.s);
+	const double rf = rp.f;
 	int32_t sq = 0;
 	int8_t* out = a.out_stream + (size_t)oidx * H;
 #pragma unroll
@@ -224,7 +217,7 @@ __global__ __launch_bounds__(512) void k_residual_gemv(GemmArgs g, sslm_launch::
 		if (lead && rl == 0) set_status(a.status, slot, a.layer, st);
 		ok = false;
 	}
-	const double nf = requant_factor(np.r, np.s);
+	const double nf = np.f;
 #pragma unroll
 	for (int k = 0; k < EP; ++k) {
 		const int el = rl + k * RT;
@@ -328,7 +321,7 @@ __global__ __launch_bounds__(64 * kCW) void k_funnel_gemv(GemmArgs g, sslm_launc
 			}
 			if (ok) a.out_scale[r] = plan.out;
 		}
-		const double f = requant_factor(plan.r, plan.s);
+		const double f = plan.f;
 #pragma unroll
 		for (int k = 0; k < CPW; ++k) {
 			const int e = 2 * ((int)threadIdx.x + k * 64 * kCW);
@@ -408,7 +401,7 @@ __global__ __launch_bounds__(512) void k_act_gemv(GemmArgs g, sslm_launch::ActAr
 			if (st0[r] == 0 && st != kOk) set_status(a.status, slot[r], a.layer, st);
 			if (ok) a.act_scale[r] = plan.out;
 		}
-		const double f = requant_factor(plan.r, plan.s);
+		const double f = plan.f;
 #pragma unroll
 		for (int k = 0; k < CPW; ++k) {
 			const int e = 2 * ((int)threadIdx.x + k * 512);

@@ -328,6 +328,7 @@ enum FwdStatus : int32_t {
 struct FunnelPlan {
 	int64_t r;
 	int s;
+	double f;  // requant_factor(r, s)
 	Scale out;
 };
 
@@ -335,26 +336,31 @@ struct FunnelOut {
 	int32_t st;
 	int32_t s;
 	int64_t r;
+	double f;
 	Scale out;
 };
 
 // reciprocal_div for a normalized dn in [2^30, 2^31), the only divisors a funnel plan has.  On the
 // GPU the estimate of 2^62 / dn is the hardware double reciprocal refined by one Newton step
-// (relative error near 2^-50, so within one of the quotient, which lies in (2^31, 2^32]) and
-// converted with one unsigned 32-bit conversion (it saturates at 2^32 - 1 only for dn = 2^30,
-// which the first correction step lifts to 2^32); the reference's two correction steps follow.
+// (relative error near 2^-50), rounded to an integer y: at most 1/2 + 2^-17 from the quotient, which lies
+// in (2^31, 2^32].  2^62 - y dn is then below 2^31 in magnitude, so one fma gives it exactly, and one
+// step of the reference's correction rule finishes it, in full-rate double operations (two
+// steps on 64-bit products were 66 instructions of a plan that runs cold, three plans a row).
 // Checked equal to reciprocal_div for every dn in [2^30, 2^31) by tests/reciprocal_norm_check.
-SSLM_HD int64_t reciprocal_norm(int64_t dn) {
+SSLM_HD double reciprocal_norm_d(double dd) {
 #if defined(__HIP_DEVICE_COMPILE__)
-	const double dd = (double)dn;
 	double r = __builtin_amdgcn_rcp(dd);
 	r = fma(r, fma(-dd, r, 1.0), r);
-	int64_t y = (int64_t)__double2uint_rz(4611686018427387904.0 * r);
-	for (int i = 0; i < 2; ++i) {
-		const int64_t res2 = (((int64_t)1 << 62) - y * dn) * 2;
-		y += res2 >= dn ? 1 : (res2 < -dn ? -1 : 0);
-	}
-	return y;
+	const double y = rint(4611686018427387904.0 * r), res2 = 2.0 * fma(-y, dd, 4611686018427387904.0);
+	return y + (res2 >= dd ? 1.0 : (res2 < -dd ? -1.0 : 0.0));
+#else
+	return (double)reciprocal_div((int64_t)dd);
+#endif
+}
+SSLM_HD int64_t reciprocal_norm(int64_t dn) {
+#if defined(__HIP_DEVICE_COMPILE__)
+	const double y = reciprocal_norm_d((double)(uint32_t)dn);  // in (2^31, 2^32]
+	return (int64_t)__double2uint_rz(y - 2147483648.0) + 2147483648ll;
 #else
 	return reciprocal_div(dn);
 #endif
@@ -371,7 +377,7 @@ SSLM_HD FunnelOut funnel_plan_v(uint64_t d_prime, int n_in, Scale in0, Scale in1
 	const bool ok_d = d <= ((uint64_t)1 << 31);
 	int s;
 	const int64_t dn = normalize_scale((int64_t)(ok_d ? d : 1), &s);
-	const int64_t r = reciprocal_norm(dn);
+	const double rd = reciprocal_norm_d((double)(uint32_t)dn);
 	Scale run = site;
 	bool ok_mid = true;
 	if (n_in > 0) {
@@ -389,7 +395,8 @@ SSLM_HD FunnelOut funnel_plan_v(uint64_t d_prime, int n_in, Scale in0, Scale in1
 	o.st = !ok_in ? kCarriedScaleMantissaOutOfDomain
 	              : (!ok_d ? kChainInputOutOfDomain : (ok_mid && ok1 && ok2 ? kOk : kCarriedScaleMantissaOutOfDomain));
 	o.s = s;
-	o.r = r;
+	o.r = (int64_t)rd;
+	o.f = ldexp(rd * 127.0, s - 62);  // exact: 127 r < 2^39
 	o.out = run;
 	return o;
 }
@@ -401,6 +408,7 @@ SSLM_HD int32_t funnel_plan(uint64_t d_prime, const Scale* incoming, int n_in, S
 	if (o.st == kOk) {
 		plan->r = o.r;
 		plan->s = o.s;
+		plan->f = o.f;
 		plan->out = o.out;
 	}
 	return o.st;
@@ -466,7 +474,8 @@ SSLM_COLD Landing landing_rescale_cold(int64_t branch, int64_t m_a, int64_t r_t,
 
 // landing_rescale for the residual site's operands (|branch| <= 127 code, |m_a| < 2^31 + 1,
 // r_t < 2^33) on 64-bit halves when the composed exponent k is non-negative; every other case
-// takes the general 128-bit path above.  Same outputs bit for bit.
+// takes the general 128-bit path above.  Same outputs bit for bit.  (The residual's kernels use
+// residual_land; this is the form it is checked against.)
 SSLM_HD int64_t landing_small(int64_t branch, int64_t m_a, int64_t r_t, int64_t k, bool* clamped, bool* exceeded) {
 	const uint64_t ab = branch < 0 ? (uint64_t)0 - (uint64_t)branch : (uint64_t)branch;
 	const uint64_t am = m_a < 0 ? (uint64_t)0 - (uint64_t)m_a : (uint64_t)m_a;
@@ -542,6 +551,19 @@ SSLM_HD int32_t landing_code(int64_t branch, int64_t m_a, int64_t r_t, int64_t k
 	*clamped = q > 127.0;
 	const int32_t c = (int32_t)fmin(q, 127.0);
 	return (branch < 0) != (m_a < 0) ? -c : c;
+}
+
+// The landed value of a residual branch code (landing_small), as a double; infinity where it exceeds
+// int64.  f = landing_scale(m, r_t, k).f: below 2^32 the estimate |code| f is within 2^-19 of the exact
+// magnitude, so its rounding is exact unless x + 1/2 lies within 2^-17 of an integer; there, and from
+// 2^32 on, the exact form runs out of line.
+SSLM_HD double residual_land(int32_t code, int64_t m, int64_t r_t, int64_t k, double f) {
+	const double x = (double)(code < 0 ? -code : code) * f, y = x + 0.5, q = floor(y), d = y - q;
+	if (!(x < 0x1p32) || d < 0x1p-17 || d > 1.0 - 0x1p-17) {
+		const Landing l = landing_rescale_cold(code, m, r_t, k);
+		return l.exceeded ? (double)INFINITY : (double)l.raw;
+	}
+	return (code < 0) != (m < 0) ? -q : q;
 }
 
 // forward_sites.cpp:399-408

@@ -1843,7 +1843,7 @@ __global__ __launch_bounds__(kRowBlock) void k_embed(const int32_t* tokens, cons
 		return;
 	}
 	int8_t* out = out_codes + (size_t)out_idx[t] * H;
-	for (int i = threadIdx.x; i < H; i += kRowBlock) out[i] = requant_code_f(row[i], requant_factor(plan.r, plan.s));
+	for (int i = threadIdx.x; i < H; i += kRowBlock) out[i] = requant_code_f(row[i], plan.f);
 	if (threadIdx.x == 0) out_scale[scale_idx[t]] = plan.out;
 }
 
@@ -2043,7 +2043,7 @@ __device__ __forceinline__ int32_t rmsnorm_regs(const int32_t (&h)[EPT], const i
 	const int32_t st = funnel_plan(mx, nullptr, 0, site, &plan);
 	if (st != kOk) return st;
 	KT(13);
-	const double f = requant_factor(plan.r, plan.s);
+	const double f = plan.f;
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) {
 		const int i = threadIdx.x + k * BS;
@@ -2236,7 +2236,7 @@ __global__ __launch_bounds__(BS) void k_qkv_post(sslm_launch::QkvPostArgs a) {
 	}
 	// q: codes of pair (2i, 2i+1), rotated, clamped; K/V: to the staging row (prefill spans: until every
 	// token's q funnel has passed) or the pool
-	const double qfac = requant_factor(plan.r, plan.s);
+	const double qfac = plan.f;
 	char2* qo = (char2*)(a.q_rot + (size_t)t * H);
 	int8_t* stage = a.kv_stage ? a.kv_stage + (size_t)t * 2 * KVH : nullptr;
 	int8_t* blk = a.kv_pool + (int64_t)ti.block * a.block_bytes;
@@ -2410,7 +2410,7 @@ __global__ __launch_bounds__(BS) void k_funnel(sslm_launch::FunnelArgs a) {
 #pragma unroll
 		for (int k = 0; k < EPT; ++k) {
 			const int i = threadIdx.x + k * BS;
-			if (i < N) out[i] = requant_code_f(fv[k], requant_factor(plan.r, plan.s));
+			if (i < N) out[i] = requant_code_f(fv[k], plan.f);
 		}
 		return;
 	}
@@ -2453,7 +2453,7 @@ __global__ __launch_bounds__(BS) void k_funnel(sslm_launch::FunnelArgs a) {
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) {
 		const int i = threadIdx.x + k * BS;
-		if (i < N) out[i] = requant_code_f(f[k], requant_factor(plan.r, plan.s));
+		if (i < N) out[i] = requant_code_f(f[k], plan.f);
 	}
 	if (threadIdx.x == 0) a.out_scale[t] = plan.out;
 }
@@ -2464,7 +2464,6 @@ template <int BS, int EPT, int RS>
 __global__ __launch_bounds__(BS) void k_residual_norm(sslm_launch::ResidualArgs a) {
 	__shared__ uint32_t s_b[BS / 64], s_r[BS / 64], s_n[BS / 64];
 	__shared__ int32_t s_ss[BS / 64];
-	__shared__ double land[256];  // landed branch value per branch code (code + 127)
 	__shared__ int32_t s_st;
 	const int t = blockIdx.x, H = a.H;
 	KT(0);
@@ -2538,12 +2537,10 @@ __global__ __launch_bounds__(BS) void k_residual_norm(sslm_launch::ResidualArgs 
 		return;
 	}
 	KT(2);
-	// The landed value depends on the branch code alone (forward_sites.cpp:513-653 with the
-	// row's scales fixed), so the 255 possible values are tabulated, one per thread;
-	// infinity marks a code whose landing exceeds int64.  Doubles hold every value the residual funnel
-	// accepts (at most 2^31) exactly.
+	// The landed value of each branch code (forward_sites.cpp:513-653); infinity marks one that exceeds
+	// int64.  Doubles hold every value the residual funnel accepts (at most 2^31) exactly.
 	int32_t code[EPT];
-	const double bfac = requant_factor(bplan.r, bplan.s);
+	const double bfac = bplan.f;
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) code[k] = requant_code_f(bf[k], bfac);
 	if (a.branch_tap.codes) {
@@ -2554,18 +2551,12 @@ __global__ __launch_bounds__(BS) void k_residual_norm(sslm_launch::ResidualArgs 
 		}
 		if (threadIdx.x == 0) a.branch_tap.scale[t] = bplan.out;
 	}
-	if (threadIdx.x < 255) {
-		const int64_t r_h = reciprocal_fast(ss.m);
-		const int64_t kx = composed_exponent(bplan.out.e, ss.e);
-		bool cl, ex;
-		const int64_t rec = landing_small((int64_t)threadIdx.x - 127, bplan.out.m, r_h, kx, &cl, &ex);
-		land[threadIdx.x] = ex ? (double)INFINITY : (double)rec;
-	}
-	__syncthreads();
+	const int64_t r_h = reciprocal_fast(ss.m), kx = composed_exponent(bplan.out.e, ss.e);
+	const double lf = landing_scale(bplan.out.m, r_h, kx).f;
 	double w[EPT], mxd = 0.0;
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) {
-		w[k] = (int)threadIdx.x + k * BS < H ? land[code[k] + 127] + (double)sv[k] : 0.0;
+		w[k] = (int)threadIdx.x + k * BS < H ? residual_land(code[k], bplan.out.m, r_h, kx, lf) + (double)sv[k] : 0.0;
 		mxd = fmax(mxd, fabs(w[k]));
 	}
 	const uint32_t mx = blk_max32<BS>(mxd == (double)INFINITY ? kBad32 : sat_u32_d(mxd), s_r);
@@ -2579,7 +2570,7 @@ __global__ __launch_bounds__(BS) void k_residual_norm(sslm_launch::ResidualArgs 
 	KT(4);
 	int8_t* out = a.out_stream + (size_t)oidx * H;
 	int32_t c[EPT];
-	const double rfac = requant_factor(rplan.r, rplan.s);
+	const double rfac = rplan.f;
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) {
 		const int i = threadIdx.x + k * BS;
@@ -2697,8 +2688,8 @@ void k_mlp_act(sslm_launch::ActArgs a) {
 	int32_t gc[EPT], uc[EPT];
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) {
-		gc[k] = requant_code_f(gf[k], requant_factor(gp.r, gp.s));
-		uc[k] = requant_code_f(uf[k], requant_factor(up.r, up.s));
+		gc[k] = requant_code_f(gf[k], gp.f);
+		uc[k] = requant_code_f(uf[k], up.f);
 	}
 	if (a.gate_tap.codes) tap_gate_up_impl<BS, EPT>(a, t, 0, I, gc, uc, gp.out, up.out, true);
 	__syncthreads();
@@ -2723,7 +2714,7 @@ void k_mlp_act(sslm_launch::ActArgs a) {
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) {
 		const int i = threadIdx.x + k * BS;
-		if (i < I) act[i] = requant_code_f(w[k], requant_factor(ap.r, ap.s));
+		if (i < I) act[i] = requant_code_f(w[k], ap.f);
 	}
 	if (threadIdx.x == 0) a.act_scale[t] = ap.out;
 }
@@ -2792,8 +2783,8 @@ __global__ __launch_bounds__(BS) void k_mlp_act_s1(sslm_launch::ActArgs a, int p
 	int32_t gc[EPT], uc[EPT];
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) {
-		gc[k] = requant_code_f(gf[k], requant_factor(gp.r, gp.s));
-		uc[k] = requant_code_f(uf[k], requant_factor(up.r, up.s));
+		gc[k] = requant_code_f(gf[k], gp.f);
+		uc[k] = requant_code_f(uf[k], up.f);
 	}
 	if (a.gate_tap.codes) tap_gate_up_impl<BS, EPT>(a, t, j0, j1, gc, uc, gp.out, up.out, sl == 0);
 	__syncthreads();
@@ -2850,7 +2841,7 @@ __global__ __launch_bounds__(BS) void k_mlp_act_s2(sslm_launch::ActArgs a, int p
 #pragma unroll
 	for (int k = 0; k < EPT; ++k) {
 		const int i = j0 + threadIdx.x + k * BS;
-		if (i < j1) act[i] = requant_code_f(w[k], requant_factor(ap.r, ap.s));
+		if (i < j1) act[i] = requant_code_f(w[k], ap.f);
 	}
 	if (threadIdx.x == 0 && sl == 0) a.act_scale[t] = ap.out;
 }
@@ -3015,8 +3006,8 @@ __global__ __launch_bounds__(BS) void k_attention(sslm_launch::AttnArgs a) {
 			}
 			if (st == kOk && i < PAIRS) {  // q codes and RoPE(q) of pair i
 				int64_t xr, yr;
-				const int32_t x = requant_code_f(qv.x, requant_factor(plan.r, plan.s));
-				const int32_t y = requant_code_f(qv.y, requant_factor(plan.r, plan.s));
+				const int32_t x = requant_code_f(qv.x, plan.f);
+				const int32_t y = requant_code_f(qv.y, plan.f);
 				rope_pair(x, y, c, sn, &xr, &yr);
 				((char2*)s_qc)[i] = make_char2((char)clamp_code(xr), (char)clamp_code(yr));
 			}
@@ -3760,8 +3751,8 @@ __global__ __launch_bounds__(64 * NW, 1) void k_attention_group(sslm_launch::Att
 		}
 		if (st0 == kOk) {  // q codes and RoPE of the group's heads
 			int64_t xr, yr;
-			const int32_t x = requant_code_f(qv.x, requant_factor(plan.r, plan.s));
-			const int32_t y = requant_code_f(qv.y, requant_factor(plan.r, plan.s));
+			const int32_t x = requant_code_f(qv.x, plan.f);
+			const int32_t y = requant_code_f(qv.y, plan.f);
 			rope_pair(x, y, cq, sq, &xr, &yr);
 			*(char2*)&s_qc[qr][2 * qj] = make_char2((char)clamp_code(xr), (char)clamp_code(yr));
 		}

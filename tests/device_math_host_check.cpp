@@ -4,6 +4,7 @@
 // per-element softmax -- must equal the reference restatements bit for bit.  Built and run
 // by tests/test_device_math_host.py; prints "ok" and exits 0 when every case agrees.
 #include <math.h>
+#include <cmath>
 #include <stdio.h>
 
 #include <random>
@@ -132,6 +133,22 @@ int main(int argc, char** argv) {
 			EXPECT(requant_code_f(x, requant_factor(r, s)) == or_requant_code_wide(x, r, s), "tie %lld %d", (long long)x, s);
 			EXPECT(or_requant_code_wide(x, r, s) == (sg ? -64 : 64), "tie rounds away from zero");
 		}
+	// residual landing by double estimate, values at and beside half-integers included
+	for (long i = 0; i < N * 4; ++i) {
+		const int64_t code = uni(-127, 127);
+		int64_t m = uni(1LL << 30, (1LL << 31) - 1) * (rng() % 8 ? 1 : -1), r_t = uni(1LL << 31, 1LL << 32), k = uni(30, 75);
+		if (i % 4 == 0) {
+			m = (1LL << 30) + (i % 8 ? 0 : uni(-2, 2));
+			r_t = (1LL << 32) + (i % 8 ? uni(-2, 2) : 0);
+			k = uni(62, 72);
+		}
+		if (i % 64 == 7) k = uni(-140, 140);
+		bool cl, ex;
+		const int64_t want = landing_small(code, m, r_t, k, &cl, &ex);
+		const double got = residual_land((int32_t)code, m, r_t, k, landing_scale(m, r_t, k).f);
+		EXPECT(ex ? std::isinf(got) : got == (double)want, "%lld %lld %lld %lld: %g %lld", (long long)code, (long long)m, (long long)r_t,
+		       (long long)k, got, (long long)want);
+	}
 	// landed K/V codes by double estimate: every exponent band, values at and beside half-integers, and
 	// operands whose product or quotient passes the estimate's domain
 	for (long i = 0; i < N * 4; ++i) {
