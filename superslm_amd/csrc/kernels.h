@@ -205,8 +205,9 @@ struct QkvPostArgs {
 	uint32_t* sat_stage;
 };
 void qkv_post(const QkvPostArgs& a, hipStream_t s);
-// (unless tiled_attention_staged()) Writes the staged K/V rows of a prefill span into the pool and adds the clamp counts, unless
-// the slot's status holds a refusal; always clears sat_stage.
+// Writes the staged K/V rows of a prefill span into the pool and adds the clamp counts, unless
+// the slot's status holds a refusal; always clears sat_stage.  Not launched where
+// tiled_attention_staged(): the attention commits the rows itself.
 void kv_commit(const QkvPostArgs& a, hipStream_t s);
 
 struct AttnArgs {
