@@ -166,7 +166,9 @@ __global__ __launch_bounds__(512) void k_residual_gemv(GemmArgs g, sslm_launch::
 	}
 	mx = row_max<NW>(mx, s_m[0]);
 	FunnelPlan bp{}, rp{}, np{};
-	bool ok = status0 == 0;
+	// Any block may report a bias refusal of the layer after a.layer at its end, before a late block (block
+	// 0 too, which commits this layer's row) has read the word: only refusals up to a.layer count here.
+	bool ok = !refused_through(status0, a.layer);
 	int32_t st = funnel_plan(mx, &bin, 1, a.branch_site, &bp);
 	if (st == kOk && !fits_i32(ss.m)) st = kCarriedScaleMantissaOutOfDomain;
 	if (ok && st != kOk) {

@@ -325,6 +325,11 @@ enum FwdStatus : int32_t {
 // and the left-associated fold of incoming factors, the site constant and (Dn, -s).
 // `d_prime` is the row's max |x| with the all-zero guard applied.  Returns a status; on Ok the
 // per-element codes are requant_code_small(x, r, s).
+// Status words, (layer << 8) | code of a slot's first refusal.  refused_through: whether the word holds a
+// refusal of `layer` or an earlier one.
+SSLM_HD int32_t status_word(int32_t layer, int32_t st) { return (layer << 8) | st; }
+SSLM_HD bool refused_through(int32_t word, int32_t layer) { return word != 0 && (word >> 8) <= layer; }
+
 struct FunnelPlan {
 	int64_t r;
 	int s;

@@ -110,7 +110,7 @@ struct RawIn {
 
 // Status word: the first rejection per sequence slot wins.
 __device__ __forceinline__ void set_status(int32_t* status, int32_t slot, int32_t layer, int32_t st) {
-	if (st != kOk) atomicCAS(&status[slot], 0, (layer << 8) | st);
+	if (st != kOk) atomicCAS(&status[slot], 0, status_word(layer, st));
 }
 
 // Attention runs its heads in parallel, but the reference runs them in order and reports the

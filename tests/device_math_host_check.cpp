@@ -226,6 +226,12 @@ int main(int argc, char** argv) {
 			for (int j = 0; j < n; ++j) EXPECT(requant_code_f(row[j], f) == codes[j], "code f");
 		}
 	}
+	// status words: a refusal counts at its own layer and at every later one, and no word at none
+	for (int l = 0; l < 80; ++l)
+		for (int at = 0; at < 80; ++at)
+			for (int c : {(int)kChainInputOutOfDomain, (int)kBiasReconcileProductOutOfDomain})
+				EXPECT(refused_through(status_word(at, c), l) == (at <= l), "status word of layer %d at %d", at, l);
+	for (int l = 0; l < 80; ++l) EXPECT(!refused_through(0, l), "no refusal at %d", l);
 	// softmax row as the attention kernel computes it (constants, gate, per-element i-exp, Q15)
 	int64_t ln2_q, b_q, ca_q;
 	or_iexp_pinned(&ln2_q, &b_q, &ca_q);
