@@ -148,6 +148,9 @@ int packed_planes(int M, int N, int K);
 // when g.wp is set and they take the launch, else gemv_plan's.  1 = a single plane, 0 = no decode
 // GEMV takes the launch.
 int gemv_raw_splits(const GemmArgs& g);
+// whether a decode step of M tokens runs the q|k|v post-processing inside its attention (`packed`: the
+// projection has its packed copy)
+bool decode_fused_ok(int M, int H, int NKV, int KVH, int64_t cap, bool packed);
 // bytes of the packed decode copy of an [N, K] matrix (whole 16-row tiles)
 size_t packed_bytes(int N, int K);
 // writes the packed decode copy of w [N, K] (K % 128 == 0) into wp

@@ -4996,6 +4996,19 @@ bool grouped_attention_chosen(int M, int NKV, int64_t cap) {
 	return M * NKV >= 64 && cap >= 1024;
 }
 
+// Up to 64 tokens always.  Past them
+// - a packed GEMV has to write the projection with its epilogue: in an unsplit prefill GEMM (36 tiles of
+//   128 x 128 at the 7B shape) it costs more than the launch saved (3 layers, 96 and 128 sequences
+//   794 and 873 us a step against 720 and 805 with raw planes and qkv_post);
+// - the grouped kernel, which holds one block per CU, has to run in one round: 100 sequences, one layer's
+//   projection, post-processing and attention, 100 blocks 29.5 against 46.9 us, 200 blocks 27.5 against 33.1
+//   (300 positions), but 400 blocks 43.2 against 44.8 (and 3 us slower at 8 positions), 1,600 blocks 112.8 against 59.5.
+bool decode_fused_ok(int M, int H, int NKV, int KVH, int64_t cap, bool packed) {
+	if (gemv_eligible(M, H)) return true;
+	return packed && H <= 4096 && packed_planes(M, H + 2 * KVH, H) == 1 &&
+	       (!grouped_attention_chosen(M, NKV, cap) || M * NKV <= device_cus());
+}
+
 void attention_decode(const AttnArgs& a, hipStream_t s) {
 	if (grouped_attention_chosen(a.M, a.NKV, a.cap)) {
 		bool done = false;

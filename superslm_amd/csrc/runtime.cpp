@@ -831,7 +831,8 @@ void run_layers(sslm_model m, Track& w, int M, StreamRef st, int l0, int l1, ssl
 		sslm_launch::rmsnorm(a, M, H, w.tok, m->status, l0, s);
 		ck(hipGetLastError());
 	}
-	const bool fused = decode && M <= kTrackTokens && H % 128 == 0 && fused_attention_enabled();
+	const bool fused = decode && fused_attention_enabled() &&
+	                   sslm_launch::decode_fused_ok(M, H, m->NKV, KVH, m->cap, m->layers[l0].p_qkv != nullptr);
 	const bool staged_attn = !decode && w.kv_stage && sslm_launch::tiled_attention_staged(M, m->NKV, m->NH);
 	const bool dbg = dbg_on(m, M);
 	// a few sequences: the context and activation funnels run inside the GEMVs that read their codes, for

@@ -73,6 +73,15 @@ int main() {
 	qa.M = 1;
 	qa.H = 1 << 20;
 	expect(refuses([&] { qkv_post(qa, nullptr); }), "qkv_post row too long");
+	// the fused decode attention past 64 rows: where a packed GEMV writes the projection and the grouped
+	// kernel (caps from 1,024) runs in one round of one block per CU (256 without a GPU)
+	const int cus = device_cus();
+	expect(decode_fused_ok(64, 3584, 4, 512, 4608, true) && decode_fused_ok(64, 3584, 4, 512, 4608, false), "fused, 64 rows");
+	expect(!decode_fused_ok(65, 3584, 4, 512, 4608, true) && !decode_fused_ok(128, 3584, 4, 512, 64, true), "not fused, depth");
+	expect(decode_fused_ok(65, 1536, 2, 256, 1024, true) && decode_fused_ok(cus / 2, 1536, 2, 256, 1024, true), "fused, one round");
+	expect(!decode_fused_ok(65, 1536, (cus + 64) / 65, 256, 1024, true), "not fused, two rounds of the grouped kernel");
+	expect(decode_fused_ok(128, 1024, 16, 1024, 512, true), "fused, one block per head");
+	expect(!decode_fused_ok(65, 1536, 2, 256, 1024, false) && !decode_fused_ok(129, 1536, 1, 128, 1024, true), "not fused, no packed launch");
 	if (bad) return 1;
 	printf("ok\n");
 	return 0;

@@ -71,3 +71,19 @@ def test_packed_rows_match_oracle(shape, batch, length, hip_lib, oracle_lib):
     assert got[0] == want[0], "tokens differ"
     for i in range(batch):
         assert np.array_equal(got[1][i], want[1][i]), f"KV of sequence {i} differs"
+
+
+@pytest.mark.parametrize("kv_heads,batch", [(2, 65), (2, 128), (4, 65), (4, 128)])
+def test_fused_decode_rule_matches_oracle(kv_heads, batch, hip_lib, oracle_lib):
+    """Past 64 sequences at a cap that takes the grouped decode attention: its blocks in one round of the
+    CUs (two KV heads: the post-processing inside the attention) and in two (four: raw planes)."""
+    sm = build_synthetic(ModelConfig(hidden=256, layers=2, heads=4, kv_heads=kv_heads, head_dim=64, inter=320, vocab=512,
+                                     context_cap=1024, tie_embeddings=True, with_bias=True), seed=29)
+    rng = np.random.default_rng(batch + kv_heads)
+    prompts = [rng.integers(0, sm.config.vocab, size=1) for _ in range(batch)]
+    want = _oracle(oracle_lib, sm, prompts, 3)
+    print(f"case fused rule kv_heads={kv_heads} batch={batch}", flush=True)
+    got = _hip(hip_lib, sm, prompts, 3)
+    assert got[0] == want[0], "tokens differ"
+    for i in range(batch):
+        assert np.array_equal(got[1][i], want[1][i]), f"KV of sequence {i} differs"
