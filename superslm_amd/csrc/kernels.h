@@ -360,7 +360,9 @@ struct ActArgs {
 	SiteTap gate_tap, up_tap;  // the gate / up funnels' codes and scales
 };
 constexpr int kMaxActSlices = 16;
-constexpr int kMaxSlicedActRows = 128;  // rows the sliced form's buffers hold
+// rows the sliced form's buffers hold; past them one block per row is the faster form (a 1.5B decode step of
+// 72, 100 and 128 sequences, sliced against whole rows: 2.53 / 2.47, 2.75 / 2.67, 2.95 / 2.78 ms)
+constexpr int kMaxSlicedActRows = 64;
 void mlp_act(const ActArgs& a, hipStream_t s);
 // The same step on every row cut into column slices, one block per (row, slice), in two
 // launches: gate and up funnels, SiLU products and per-slice maxima; then the act funnel over the

@@ -34,10 +34,9 @@ constexpr int kMaxTokens = 512;      // tokens per launch sequence (prefill chun
 constexpr int kTracks = 4;           // concurrent token groups of one decode step
 constexpr int kTrackTokens = 128;    // tokens per launch on tracks 1..kTracks-1
 constexpr int kSlotCapacity = 1024;  // live sequences per model
-// A decode unit (at most kTrackTokens rows) takes the sliced SiLU at any size (1.5B, 72 and 128
-// sequences: a burst 250.5 -> 246.9, 386.6 -> 383.0 ms); a prefill span only while it is this short: 100
-// prompts of 4-12 tokens 295.4 -> 292.6 ms, while at 65 and 96 tokens one block per row is faster (8 prompts
-// 23.2 against 23.5 and 23.6 against 24.9 ms).
+// A decode unit takes the sliced SiLU up to kMaxSlicedActRows rows; a prefill span only while it is this
+// short: 100 prompts of 4-12 tokens 295.4 -> 292.6 ms, while at 65 and 96 tokens one block per row is faster
+// (8 prompts 23.2 against 23.5 and 23.6 against 24.9 ms).
 constexpr int kSlicedActPrefillRows = 32;
 
 struct HipError {

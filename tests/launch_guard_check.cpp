@@ -82,6 +82,16 @@ int main() {
 	expect(!decode_fused_ok(65, 1536, (cus + 64) / 65, 256, 1024, true), "not fused, two rounds of the grouped kernel");
 	expect(decode_fused_ok(128, 1024, 16, 1024, 512, true), "fused, one block per head");
 	expect(!decode_fused_ok(65, 1536, 2, 256, 1024, false) && !decode_fused_ok(129, 1536, 1, 128, 1024, true), "not fused, no packed launch");
+	// the sliced SiLU up to 64 rows
+	ActArgs sl{};
+	sl.I = 8960;
+	sl.prod = &f[0];
+	sl.act_maxpart = (uint32_t*)f;
+	sl.gu_scale = (Scale*)fold;
+	sl.M = 64;
+	expect(mlp_act_sliced_ok(sl), "sliced SiLU, 64 rows");
+	sl.M = 65;
+	expect(!mlp_act_sliced_ok(sl), "no sliced SiLU, 65 rows");
 	if (bad) return 1;
 	printf("ok\n");
 	return 0;
