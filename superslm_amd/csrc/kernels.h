@@ -155,6 +155,7 @@ bool decode_fused_ok(int M, int H, int NKV, int KVH, int64_t cap, bool packed);
 size_t packed_bytes(int N, int K);
 // writes the packed decode copy of w [N, K] (K % 128 == 0) into wp
 void pack_gemv(const int8_t* w, int N, int K, int8_t* wp, hipStream_t s);
+bool gemm_lds_loads_ok(const GemmArgs& g);  // past 64 rows: the operands' alignment admits direct loads to LDS
 bool wide_gemm_ok(const GemmArgs& g);  // the prefill launch takes the 256 x 160-tile kernel
 // launch shape of the prefill GEMM; `split_ok` as for gemv_plan
 PrefillPlan prefill_plan(int M, int N, int K, bool split_ok);

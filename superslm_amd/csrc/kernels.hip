@@ -4610,6 +4610,18 @@ static bool narrow_funnel_ok(const GemmArgs& g) {
 	return g.M > 64 && g.splits <= 1 && g.K % 16 == 0 && funnel_segments_ok(g) && narrow_tiles(g) <= kNarrowFunnelMaxTiles;
 }
 
+// The kernels past 64 rows fetch their operands straight into LDS, 16 bytes a lane, from rows of 16-byte
+// alignment.  The GEMM entries ask for no alignment: an operand at another address takes k_gemm_tiled,
+// whose loads go through registers, where the depth is not a multiple of 128.
+bool gemm_lds_loads_ok(const GemmArgs& g) {
+	return g.K % kPBK == 0 || (((uintptr_t)g.a | (uintptr_t)g.w | (uintptr_t)g.lda) % 16 == 0);
+}
+
+static void launch_gemm_tiled(const GemmArgs& g, hipStream_t s) {
+	const dim3 grid((g.N + kBN - 1) / kBN, (g.M + kBM - 1) / kBM);
+	hipLaunchKernelGGL(k_gemm_tiled, grid, dim3(kBlock), 0, s, g);
+}
+
 void gemm(const GemmArgs& g, hipStream_t s) {
 	if (g.M <= 0 || g.N <= 0) return;
 	check_gemm_outputs(g);
@@ -4676,6 +4688,10 @@ void gemm(const GemmArgs& g, hipStream_t s) {
 	bool lora = false;
 	for (int i = 0; i < g.epi.nseg; ++i) lora = lora || g.epi.seg[i].lora_b;
 	const bool rag = g.K % kPBK != 0;
+	if (!gemm_lds_loads_ok(g)) {
+		launch_gemm_tiled(g, s);
+		return;
+	}
 	if (narrow_funnel_ok(g)) {
 		const int tiles = narrow_tiles(g);
 		if (rag) hipLaunchKernelGGL((k_gemm_narrow<true, true>), dim3(tiles), dim3(256), 0, s, g);
@@ -4707,8 +4723,7 @@ void gemm(const GemmArgs& g, hipStream_t s) {
 		}
 		return;
 	}
-	dim3 grid((g.N + kBN - 1) / kBN, (g.M + kBM - 1) / kBM);
-	hipLaunchKernelGGL(k_gemm_tiled, grid, dim3(kBlock), 0, s, g);
+	launch_gemm_tiled(g, s);
 }
 
 bool prefill_mfma_k(int K) { return K > 0 && K % kPBK == 0; }

@@ -92,6 +92,17 @@ int main() {
 	expect(mlp_act_sliced_ok(sl), "sliced SiLU, 64 rows");
 	sl.M = 65;
 	expect(!mlp_act_sliced_ok(sl), "no sliced SiLU, 65 rows");
+	// direct loads to LDS at ragged depths only from rows of 16-byte alignment
+	GemmArgs al{};
+	al.K = al.lda = 208;
+	for (int off = 0; off < 32; ++off) {
+		al.a = (const int8_t*)(uintptr_t)(4096 + off);
+		al.w = (const int8_t*)(uintptr_t)8192;
+		expect(gemm_lds_loads_ok(al) == (off % 16 == 0), "alignment of the activations");
+		al.a = (const int8_t*)(uintptr_t)4096;
+		al.w = (const int8_t*)(uintptr_t)(8192 + off);
+		expect(gemm_lds_loads_ok(al) == (off % 16 == 0), "alignment of the weights");
+	}
 	if (bad) return 1;
 	printf("ok\n");
 	return 0;

@@ -57,3 +57,19 @@ def test_ragged_requant_matches_oracle(m, n, k, hip_lib, oracle_lib):
     assert st.numpy()[rows].tolist() == st_o
     assert np.array_equal(codes.numpy()[rows], codes_o)
     assert [tuple(r) for r in me.numpy()[rows].tolist()] == scales_o
+
+
+@pytest.mark.parametrize("off_a,off_w", [(4, 0), (0, 8), (12, 4)])
+def test_ragged_operands_off_alignment(off_a, off_w, hip_lib):
+    """Operands at any 4-byte address: past 64 rows they take the tiles that load through registers."""
+    L = _lib(hip_lib)
+    dev = Device(hip_lib)
+    for m, n, k in [(65, 80, 48), (100, 208, 240), (300, 272, 1552)]:
+        a, w, _ = _inputs(m, n, k)
+        want = (a.astype(np.float64) @ w.astype(np.float64).T).astype(np.int64)
+        da = dev.upload(np.concatenate([np.zeros(off_a, np.int8), a.ravel()]))
+        dw = dev.upload(np.concatenate([np.zeros(off_w, np.int8), w.ravel()]))
+        out = dev.zeros((m, n), np.int32)
+        print(f"case ragged off alignment m={m} n={n} k={k} {off_a} {off_w}", flush=True)
+        assert L.sslm_hip_gemm_i32(da.ptr + off_a, dw.ptr + off_w, m, n, k, out.ptr) == 0
+        assert np.array_equal(out.numpy(), want)
