@@ -18,7 +18,9 @@
 //
 // The arithmetic is that of k_funnel, k_residual_norm, k_mlp_act_s2 and k_gemv_pk / k_gemv_sk, element by
 // element; block 0 writes the rows' codes, scales and refusals where those kernels do.  A row that is
-// refused, or was before, multiplies as zeros and reports nothing further.
+// refused, or was before, multiplies as zeros and reports nothing further.  (k_funnel_gemv: a block that
+// reads head_status after block 0 has resolved it multiplies the row as any other.  Either product is
+// dropped: every later kernel leaves a refused row by its status word.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -1,7 +1,8 @@
 """Decode of one to four sequences, where each funnel runs inside the GEMV that reads its codes: tokens
 and KV against the C oracle over geometries that take each kernel instance, and refusals (a
-pending token whose embedding is zero, a bias out of range at layer 1) against the same sequences
-decoded in a larger batch, whose row kernels are launches of their own."""
+pending token whose embedding is zero; at layer 1 a bias out of range, i-exp constants out of range in
+one KV group's heads, a branch that dwarfs the residual stream) against the same sequences decoded
+in a larger batch, whose row kernels are launches of their own."""
 import struct
 
 import numpy as np
@@ -74,6 +75,29 @@ def _bias_edit(m):
     m.biases["layer1.q_proj"] = (m.biases["layer1.q_proj"] * (1 << 34)).astype(np.int64)
 
 
+def _scale_edit(**shifts):
+    """Site constants of layer 0 and 1 (`l<layer>_<site>`) shifted by powers of two."""
+    def edit(m):
+        for name, shift in shifts.items():
+            key = f"layer{name[1]}.{name[3:]}"
+            sm, se = m.consts[key]
+            m.consts[key] = (sm, se + shift)
+    return edit
+
+
+# layer 1 refuses in the attention (resolved and cleared by the context funnel inside the o GEMV), or in
+# the residual after the o or down projection: a landed value past 2^31, or past int64
+EDITS = {
+    "bias": _bias_edit,
+    "attn_high": _scale_edit(l1_softmax_khead1=40),
+    "attn_low": _scale_edit(l1_softmax_khead1=-40),
+    "o_wide": _scale_edit(l1_o_proj=40),
+    "o_past_int64": _scale_edit(l0_mlp_residual=-40, l1_o_proj=40),
+    "down_wide": _scale_edit(l1_down_proj=40),
+    "down_past_int64": _scale_edit(l1_attn_residual=-40, l1_down_proj=40),
+}
+
+
 def _blobs(hip_lib, art, n, bad_at):
     """n saved sequences with a pending token each, sequence `bad_at`'s the zero-embedding one."""
     model = Model(hip_lib, art)
@@ -103,19 +127,24 @@ def _decode(model, blobs, budget, calls):
 
 
 @pytest.mark.parametrize("kind,batch,bad_at", [("zero", 1, 0), ("zero", 3, 1), ("zero", 4, 3), ("bias", 1, -1), ("bias", 4, -1),
-                                               ("clean", 4, -1)])
+                                               ("clean", 4, -1)] +
+                         [(k, b, -1) for k in EDITS if k != "bias" for b in (1, 3, 4)])
 @pytest.mark.parametrize("budget", [3, 2, 1])
 def test_chain_refusals_match_row_kernels(kind, batch, bad_at, budget, hip_lib):
-    sm = build_synthetic(SHAPES["c2"], seed=23, edit=_bias_edit if kind == "bias" else None)
+    sm = build_synthetic(SHAPES["c2"], seed=23, edit=EDITS.get(kind))
     art = with_weight_rows(sm, "embed", {BAD: np.zeros(sm.config.hidden, np.int8)}) if kind == "zero" else sm.to_array()
     model, blobs = _blobs(hip_lib, art, 6, bad_at)
     print(f"case chain refusal {kind} batch={batch} budget={budget}", flush=True)
     few = _decode(model, blobs[:batch], budget, 3)
+    again = _decode(model, blobs[:batch], budget, 3)  # in the same slots: nothing of a refusal is left behind
     many = _decode(model, blobs, budget, 3)
+    assert few == again
     assert kind == "clean" or any(st != 0 for st, _, _ in few)
     for (st, toks, saved), (st6, toks6, saved6) in zip(few, many):
         if kind == "clean" or bad_at >= 0 or st != 0:
             assert st == st6
+        if kind in EDITS:  # refused at layer 1, not before
+            assert (st == 0) == (budget == 1 and saved is few[0][2])
         assert toks == toks6[:batch]
         assert saved == saved6[:batch], "sequence state differs"
     model.close()
