@@ -189,44 +189,15 @@ SSLM_HD int64_t reciprocal_fast(int64_t dn) {
 #endif
 }
 
-// src/intmath.cpp:476-490 -- clamp(round_away(x*127*R / 2^(62-s)), +-127).
-SSLM_HD int8_t requant_code(int64_t x, int64_t r, int s) {
-	int exponent = 62 - s;
-	uint64_t ax = x < 0 ? (~(uint64_t)x + 1u) : (uint64_t)x;
-	u128 prod = (u128)ax * (uint64_t)r * 127u;
-	u128 num = prod * 2 + ((u128)1 << exponent);
-	uint64_t mag = (uint64_t)(num >> (exponent + 1));
-	if (mag > 127u) mag = 127u;
-	int32_t q = (int32_t)mag;
-	return (int8_t)(x < 0 ? -q : q);
-}
-
-// Same composite for |x| <= 2^31 (the funnel's whole accepted domain): |x|*127*R < 2^70 is
-// held as a (hi, lo) pair and the rounding shift 2^(62-s) (s in [-1, 30]) is done on 64-bit
-// halves -- mag = (prod + 2^(e-1)) >> e is the reference's (2 prod + 2^e) >> (e + 1).
-SSLM_HD int8_t requant_code_small(int64_t x, uint64_t r, int s) {
-	const int e = 62 - s;  // 32..63
-	const uint64_t ax = x < 0 ? (uint64_t)0 - (uint64_t)x : (uint64_t)x;
-	const uint64_t a = ax * 127u;  // < 2^39
-	const uint64_t lo = a * r;
-	uint64_t hi = (uint64_t)(((u128)a * r) >> 64);
-	const uint64_t lo2 = lo + ((uint64_t)1 << (e - 1));
-	hi += lo2 < lo ? 1u : 0u;
-	uint64_t mag = (lo2 >> e) | (hi << (64 - e));
-	if ((hi >> e) != 0 || mag > 127u) mag = 127u;
-	const int32_t q = (int32_t)mag;
-	return (int8_t)(x < 0 ? -q : q);
-}
-
-// requant_code_small in double arithmetic, for |x| <= 2^31 and a funnel plan's (r, s), r in
-// (2^31, 2^32] and s in [-1, 30].  The code is floor(q + 1/2), clamped to 127, for the exact
-// quotient q = |x| 127 r / 2^(62-s).  f = 127 r 2^-(62-s) is exact in a double (127 r < 2^39),
+// src/intmath.cpp:476-490 -- clamp(round_away(x 127 r / 2^(62-s)), +-127) -- in double arithmetic, for
+// |x| <= 2^31 and a funnel plan's (r, s), r in (2^31, 2^32] and s in [-1, 30].  The code is
+// floor(q + 1/2), clamped to 127, for the exact quotient q = |x| 127 r / 2^(62-s).  The plan's
+// f = 127 r 2^-(62-s) is exact in a double (127 r < 2^39),
 // so q = |x| f exactly and fma(|x|, f, 1/2) is q + 1/2 rounded once.  Rounding is monotone, so
 // m0 = floor of it is the code or, where q + 1/2 was rounded up to an integer, one more; that is
 // exactly when |x| f + (1/2 - m0) < 0, and an fma has the sign of its exact value (1/2 - m0 is exact
 // for every m0 that can be a code).  Every operation is full rate on CDNA's FP64 pipes, where the
 // 128-bit integer form takes eight quarter-rate multiplies.
-SSLM_HD double requant_factor(int64_t r, int s) { return ldexp((double)(r * 127), -(62 - s)); }
 SSLM_HD int32_t requant_mag(double a, double f) {  // a = |x|
 	const double m0 = floor(fma(a, f, 0.5));
 	const double e = fma(a, f, 0.5 - m0);
@@ -242,38 +213,6 @@ SSLM_HD int8_t requant_code_f(int64_t x, double f) {
 SSLM_HD int8_t requant_code_d(double x, double f) {
 	const int32_t c = requant_mag(fabs(x), f);
 	return (int8_t)(x < 0.0 ? -c : c);
-}
-
-// src/intmath.cpp:502-524
-SSLM_HD int64_t isqrt(int64_t n) {
-	int64_t rem = n, root = 0, bit = (int64_t)1 << 62;
-	for (int i = 0; i < 32; ++i) {
-		int64_t trial = root + bit;
-		if (rem >= trial) {
-			rem -= trial;
-			root = (root >> 1) + bit;
-		} else {
-			root >>= 1;
-		}
-		bit >>= 2;
-	}
-	return root;
-}
-
-// floor(sqrt(n)) -- the value isqrt() returns for every int64 n (0 for n <= 0) -- from a
-// double-precision estimate corrected with exact 64-bit squares.
-// The double estimate is within one of floor(sqrt(n)) for every int64 n (n rounds to a double by
-// at most 2^10, which moves the root by far less than one; the root rounds by at most 2^-21), so
-// two fixed correction steps each way replace the loops (no loop: straight-line code on the GPU;
-// (r + 1)^2 <= 3037000500^2 < 2^64 cannot wrap).
-SSLM_HD int64_t isqrt_fast(int64_t n) {
-	const uint64_t un = n > 0 ? (uint64_t)n : 0;
-	uint64_t r = (uint64_t)sqrt((double)un);
-#pragma unroll
-	for (int i = 0; i < 2; ++i) r -= r * r > un ? 1 : 0;
-#pragma unroll
-	for (int i = 0; i < 2; ++i) r += (r + 1) * (r + 1) <= un ? 1 : 0;
-	return (int64_t)r;
 }
 
 SSLM_HD int64_t sat_add64(int64_t a, int64_t b) {
@@ -321,19 +260,19 @@ enum FwdStatus : int32_t {
 	kBiasReconcileProductOutOfDomain = 24,
 };
 
-// The funnel's scale half (checked_chain_funnel.cpp:268-329): checks, the D'-derived (Dn, s, R)
-// and the left-associated fold of incoming factors, the site constant and (Dn, -s).
-// `d_prime` is the row's max |x| with the all-zero guard applied.  Returns a status; on Ok the
-// per-element codes are requant_code_small(x, r, s).
 // Status words, (layer << 8) | code of a slot's first refusal.  refused_through: whether the word holds a
 // refusal of `layer` or an earlier one.
 SSLM_HD int32_t status_word(int32_t layer, int32_t st) { return (layer << 8) | st; }
 SSLM_HD bool refused_through(int32_t word, int32_t layer) { return word != 0 && (word >> 8) <= layer; }
 
+// The funnel's scale half (checked_chain_funnel.cpp:268-329): checks, the D'-derived (Dn, s, R)
+// and the left-associated fold of incoming factors, the site constant and (Dn, -s).
+// `d_prime` is the row's max |x| with the all-zero guard applied.  Returns a status; on Ok the
+// per-element codes are requant_code_f(x, f).
 struct FunnelPlan {
 	int64_t r;
 	int s;
-	double f;  // requant_factor(r, s)
+	double f;  // 127 r 2^-(62-s)
 	Scale out;
 };
 
@@ -477,57 +416,6 @@ SSLM_COLD Landing landing_rescale_cold(int64_t branch, int64_t m_a, int64_t r_t,
 	return l;
 }
 
-// landing_rescale for the residual site's operands (|branch| <= 127 code, |m_a| < 2^31 + 1,
-// r_t < 2^33) on 64-bit halves when the composed exponent k is non-negative; every other case
-// takes the general 128-bit path above.  Same outputs bit for bit.  (The residual's kernels use
-// residual_land; this is the form it is checked against.)
-SSLM_HD int64_t landing_small(int64_t branch, int64_t m_a, int64_t r_t, int64_t k, bool* clamped, bool* exceeded) {
-	const uint64_t ab = branch < 0 ? (uint64_t)0 - (uint64_t)branch : (uint64_t)branch;
-	const uint64_t am = m_a < 0 ? (uint64_t)0 - (uint64_t)m_a : (uint64_t)m_a;
-	if (k < 0 || ab > 127u || am > ((uint64_t)1 << 31) || (uint64_t)r_t >= ((uint64_t)1 << 33))
-	{
-		const Landing l = landing_rescale_cold(branch, m_a, r_t, k);
-		*clamped = l.clamped;
-		*exceeded = l.exceeded;
-		return l.raw;
-	}
-	const bool neg = (branch < 0) != (m_a < 0);
-	const uint64_t a = ab * am;  // < 2^39
-	const uint64_t lo = a * (uint64_t)r_t;
-	const uint64_t hi = (uint64_t)(((u128)a * (uint64_t)r_t) >> 64);  // prod < 2^72
-	uint64_t qlo, qhi;
-	if (k == 0) {
-		qlo = lo;
-		qhi = hi;
-	} else if (k >= 73) {
-		qlo = 0;
-		qhi = 0;
-	} else {
-		// (prod + 2^(k-1)) >> k
-		uint64_t alo = lo, ahi = hi;
-		if (k - 1 < 64) {
-			alo = lo + ((uint64_t)1 << (k - 1));
-			ahi = hi + (alo < lo ? 1u : 0u);
-		} else {
-			ahi = hi + ((uint64_t)1 << (k - 1 - 64));
-		}
-		if (k < 64) {
-			qlo = (alo >> k) | (ahi << (64 - k));
-			qhi = ahi >> k;
-		} else {
-			qlo = ahi >> (k - 64);
-			qhi = 0;
-		}
-	}
-	const bool exc_clamp = qhi != 0 || qlo > 127;
-	const bool exc_i64 = qhi != 0 || qlo > (uint64_t)kI64Max;
-	int64_t raw = (int64_t)qlo;
-	if (neg) raw = (int64_t)(0u - (uint64_t)raw);
-	*clamped = exc_clamp || raw < -127 || raw > 127;
-	*exceeded = exc_i64;
-	return raw;
-}
-
 SSLM_HD int64_t clamp_code(int64_t v) { return v > 127 ? 127 : (v < -127 ? -127 : v); }
 
 // The landed code of a K or V value, clamp_code(landing_rescale(...)), and its clamp flag, from a
@@ -558,7 +446,7 @@ SSLM_HD int32_t landing_code(int64_t branch, int64_t m_a, int64_t r_t, int64_t k
 	return (branch < 0) != (m_a < 0) ? -c : c;
 }
 
-// The landed value of a residual branch code (landing_small), as a double; infinity where it exceeds
+// The landed value of a residual branch code (landing_rescale), as a double; infinity where it exceeds
 // int64.  f = landing_scale(m, r_t, k).f: below 2^32 the estimate |code| f is within 2^-19 of the exact
 // magnitude, so its rounding is exact unless x + 1/2 lies within 2^-17 of an integer; there, and from
 // 2^32 on, the exact form runs out of line.
@@ -569,12 +457,6 @@ SSLM_HD double residual_land(int32_t code, int64_t m, int64_t r_t, int64_t k, do
 		return l.exceeded ? (double)INFINITY : (double)l.raw;
 	}
 	return (code < 0) != (m < 0) ? -q : q;
-}
-
-// forward_sites.cpp:399-408
-SSLM_HD int64_t floor_div(int64_t a, int64_t b) {
-	int64_t q = a / b, r = a % b;
-	return (r != 0 && r < 0) ? q - 1 : q;
 }
 
 // src/intmath.cpp:782-792
@@ -774,9 +656,9 @@ SSLM_HD int32_t div_q15_small(int64_t e, double d, double inv) {
 
 // floor(v 2^32 / root) for a code v in [-128, 127] and 1 <= root < 2^24 (the RMSNorm's
 // per-code quotient, forward_sites.cpp:410-459: floor for v >= 0, -ceil(|v| 2^32 / root) below),
-// given inv = 1.0 / root.  n = v 2^32 (|n| <= 2^39) is exact in a double and the estimate n inv is
-// within 2^-12 of the quotient; q root <= |n| + root < 2^53 is exact too, so fma gives the exact
-// remainder for the one-step correction.
+// given inv within 2^-40 of 1 / root (rcp_est).  n = v 2^32 (|n| <= 2^39) is exact in a double, so
+// the estimate n inv is less than one from the quotient and its floor at most one off; q root <= |n| + root
+// < 2^53 is exact too, so fma gives the exact remainder for the one-step correction.
 SSLM_HD double norm_qd(int32_t v, double root, double inv) {
 	const double n = (double)v * 4294967296.0;
 	const double q = floor(n * inv);
@@ -811,7 +693,6 @@ SSLM_HD int64_t rms_root(int32_t ss, int32_t h) {
 	r += ((uint64_t)r + 1) * ((uint64_t)r + 1) * uh <= n ? 1u : 0u;
 	return ss > 0 && r > 1 ? r : 1;
 }
-SSLM_HD int64_t norm_fd(int32_t v, double root, double inv) { return (int64_t)norm_qd(v, root, inv); }
 
 SSLM_HD int64_t softmax_ceiling(int64_t q_b, int64_t q_c) {
 	s128 m128 = (s128)q_b * q_b + (s128)q_c;

@@ -1,6 +1,6 @@
 // Host-side check of the device integer primitives (superslm_amd/csrc/int_math.h) against
 // the C oracle (oracle/sslm_oracle.c): the GPU kernels' fast formulations -- double-estimate
-// reciprocal and division, 64-bit-half requant and landing, double-estimate isqrt, the
+// reciprocal and division, requant codes in doubles, landings by double estimate, the RMSNorm's root, the
 // per-element softmax -- must equal the reference restatements bit for bit.  Built and run
 // by tests/test_device_math_host.py; prints "ok" and exits 0 when every case agrees.
 #include <math.h>
@@ -44,6 +44,9 @@ static int exact_half_up(uint32_t a, double f) {
 	return mag > 127 ? 127 : (int)mag;
 }
 
+// a funnel plan's factor for (r, s): 127 r 2^-(62-s), exact
+static double factor(int64_t r, int s) { return ldexp((double)(r * 127), -(62 - s)); }
+
 int main(int argc, char** argv) {
 	const long N = argc > 1 ? atol(argv[1]) : 200000;
 	std::mt19937_64 rng(20261201);
@@ -63,17 +66,6 @@ int main(int argc, char** argv) {
 		const int64_t d = i % 3 ? uni(1, 1LL << (int)uni(0, 62)) : uni(1, 300);
 		EXPECT(div_floor_pos(n, d) == n / d, "%lld / %lld", (long long)n, (long long)d);
 	}
-	// isqrt
-	for (long i = 0; i < N; ++i) {
-		const int bits = (int)uni(0, 63);
-		const int64_t n = bits == 63 ? uni(0, INT64_MAX) : uni(0, (int64_t)((1ULL << bits) - 1));
-		EXPECT(isqrt_fast(n) == or_isqrt(n), "%lld", (long long)n);
-	}
-	for (int64_t r = 0; r < 100000; ++r)
-		for (int64_t d = -1; d <= 1; ++d) {
-			const int64_t n = r * r + d;
-			if (n >= 0) EXPECT(isqrt_fast(n) == or_isqrt(n), "%lld", (long long)n);
-		}
 	// the RMSNorm's root
 	for (long i = 0; i < N; ++i) {
 		const int32_t h = (int32_t)(i % 3 ? uni(1, 8192) : 64 * uni(1, 128));
@@ -87,9 +79,8 @@ int main(int argc, char** argv) {
 		const int64_t dn = uni(1LL << 30, (1LL << 31) - 1);
 		const int64_t r = or_reciprocal(dn);
 		const int s = (int)uni(-1, 30);
-		EXPECT(requant_code_small(x, (uint64_t)r, s) == or_requant_code_wide(x, r, s), "%lld %lld %d", (long long)x,
-		       (long long)r, s);
-		EXPECT(requant_code_f(x, requant_factor(r, s)) == or_requant_code_wide(x, r, s), "f %lld %lld %d", (long long)x,
+		EXPECT(requant_code_f(x, factor(r, s)) == or_requant_code_wide(x, r, s), "f %lld %lld %d", (long long)x, (long long)r, s);
+		EXPECT(requant_code_d((double)x, factor(r, s)) == or_requant_code_wide(x, r, s), "d %lld %lld %d", (long long)x,
 		       (long long)r, s);
 	}
 	// the double form at the rounding boundaries: x around (n - 1/2) 2^(62-s) / (127 r) for every
@@ -106,7 +97,9 @@ int main(int argc, char** argv) {
 			if (xa < 0 || xa > (1LL << 31)) continue;
 			for (int sg = 0; sg < 2; ++sg) {
 				const int64_t x = sg ? -xa : xa;
-				EXPECT(requant_code_f(x, requant_factor(r, s)) == or_requant_code_wide(x, r, s), "edge %lld %lld %d",
+				EXPECT(requant_code_f(x, factor(r, s)) == or_requant_code_wide(x, r, s), "edge %lld %lld %d",
+				       (long long)x, (long long)r, s);
+				EXPECT(requant_code_d((double)x, factor(r, s)) == or_requant_code_wide(x, r, s), "edge d %lld %lld %d",
 				       (long long)x, (long long)r, s);
 			}
 		}
@@ -130,7 +123,7 @@ int main(int argc, char** argv) {
 	for (int s = -1; s <= 29; ++s)
 		for (int sg = 0; sg < 2; ++sg) {
 			const int64_t r = 1LL << 32, x = (sg ? -1 : 1) * (1LL << (29 - s));
-			EXPECT(requant_code_f(x, requant_factor(r, s)) == or_requant_code_wide(x, r, s), "tie %lld %d", (long long)x, s);
+			EXPECT(requant_code_f(x, factor(r, s)) == or_requant_code_wide(x, r, s), "tie %lld %d", (long long)x, s);
 			EXPECT(or_requant_code_wide(x, r, s) == (sg ? -64 : 64), "tie rounds away from zero");
 		}
 	// residual landing by double estimate, values at and beside half-integers included
@@ -144,7 +137,7 @@ int main(int argc, char** argv) {
 		}
 		if (i % 64 == 7) k = uni(-140, 140);
 		bool cl, ex;
-		const int64_t want = landing_small(code, m, r_t, k, &cl, &ex);
+		const int64_t want = landing_rescale(code, m, r_t, k, &cl, &ex);
 		const double got = residual_land((int32_t)code, m, r_t, k, landing_scale(m, r_t, k).f);
 		EXPECT(ex ? std::isinf(got) : got == (double)want, "%lld %lld %lld %lld: %g %lld", (long long)code, (long long)m, (long long)r_t,
 		       (long long)k, got, (long long)want);
@@ -182,7 +175,7 @@ int main(int argc, char** argv) {
 		const int64_t e_a = uni(-150, 50), e_t = uni(-150, 50);
 		const int64_t k = composed_exponent(e_a, e_t);
 		bool cl1, ex1;
-		const int64_t v1 = landing_small(branch, m_a, r_t, k, &cl1, &ex1);
+		const int64_t v1 = landing_rescale(branch, m_a, r_t, k, &cl1, &ex1);
 		uint64_t sat = 0;
 		int ex2 = 0;
 		const int64_t v2 = or_landing_rescale(branch, m_a, r_t, e_a, e_t, &sat, &ex2);
@@ -221,9 +214,9 @@ int main(int argc, char** argv) {
 		EXPECT(st == ost, "status %d vs %d", st, ost);
 		if (st == 0 && ost == 0) {
 			EXPECT(plan.out.m == out.m && plan.out.e == out.e, "scale");
-			for (int j = 0; j < n; ++j) EXPECT(requant_code_small(row[j], (uint64_t)plan.r, plan.s) == codes[j], "code");
-			const double f = requant_factor(plan.r, plan.s);
-			for (int j = 0; j < n; ++j) EXPECT(requant_code_f(row[j], f) == codes[j], "code f");
+			EXPECT(plan.f == factor(plan.r, plan.s), "factor");
+			for (int j = 0; j < n; ++j) EXPECT(requant_code_f(row[j], plan.f) == codes[j], "code f");
+			for (int j = 0; j < n; ++j) EXPECT(requant_code_d((double)row[j], plan.f) == codes[j], "code d");
 		}
 	}
 	// status words: a refusal counts at its own layer and at every later one, and no word at none

@@ -95,12 +95,12 @@ int main(int argc, char** argv) {
 	for (int64_t it = 0; it < (1 << 16) + N / 8; ++it) {
 		int64_t root = it < (1 << 16) ? 1 + it : 1 + (int64_t)(rng() % (1ull << 24));
 		if (it % 1009 == 0) root = (1ll << 24) - 1 - (int64_t)(rng() % 4);
-		const double rd = (double)root, inv = 1.0 / rd;
+		const double rd = (double)root, inv = rcp_est(rd);
 		for (int v = -128; v < 128; ++v) {
 			++nn;
-			const int64_t a = fd_table(v, root), b = norm_fd(v, rd, inv);
-			if (a != b) { if (bn < 10) printf("norm_fd mismatch v=%d root=%lld: %lld vs %lld\n", v, (long long)root, (long long)a, (long long)b); ++bn; }
+			const int64_t a = fd_table(v, root), b = (int64_t)norm_qd(v, rd, inv);
+			if (a != b) { if (bn < 10) printf("norm_qd mismatch v=%d root=%lld: %lld vs %lld\n", v, (long long)root, (long long)a, (long long)b); ++bn; }
 		}
 	}
-	printf("norm_fd: %ld cases, %ld mismatches\n", nn, bn);
+	printf("norm_qd: %ld cases, %ld mismatches\n", nn, bn);
 }
