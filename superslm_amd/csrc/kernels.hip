@@ -2075,13 +2075,14 @@ __global__ __launch_bounds__(BS) void k_rmsnorm(sslm_launch::RowNormArgs a, int 
 }
 
 // q funnel + RoPE(q); K/V landing, RoPE(K), KV write (forward_sites.cpp:1281-1418, :1748-1787).
-// Latency-bound, one block per token.  The row's pairs -- q, then K, then V, in the projection's column
-// order -- are spread evenly over the threads (NP each), every load is issued before the first
-// use, and the K/V landing, which does not depend on the q funnel, is computed while the q maximum is
-// reduced.  A launch fetches its instructions cold, so one landing body serves K and V
-// (128-bit landings inlined at each of eight values, 24 KB of code: 9.4-10.1 us at hidden 1536, now
-// 12 KB and 6.6-7.1; past a thousand rows of hidden 3584 the spare slots cost, 27 -> 33 us of 2 ms a layer).
-template <int BS, int NP, int RS>
+// Latency-bound, one block per token, NP pairs a thread.  Every load is issued before the first use, and
+// the K/V landing, which does not depend on the q funnel, is computed while the q maximum is reduced.  One
+// landing body by double estimate serves K and V (128-bit landings at each of eight values: 9.4-10.1 us at
+// hidden 1536, now 6.6-7.1).  Two spreads of the row over the threads, chosen in qkv_post():
+// - EQ = 0: the pairs -- q, then K, then V, in the projection's column order -- evenly; a slot may hold any;
+// - EQ > 0: q pairs in slots below EQ, K and V pairs in the others: a slot's kind is known to the compiler,
+//   and only the K/V slots hold landing operands.
+template <int BS, int NP, int EQ, int RS>
 __global__ __launch_bounds__(BS) void k_qkv_post(sslm_launch::QkvPostArgs a) {
 	__shared__ uint32_t s_red[BS / 64];
 	__shared__ int32_t s_st;
@@ -2098,11 +2099,13 @@ __global__ __launch_bounds__(BS) void k_qkv_post(sslm_launch::QkvPostArgs a) {
 	int pi[NP], hd[NP];  // pair within its head, KV head (q pairs: the first)
 	int64_t v0[NP], v1[NP], rt[NP], et[NP];
 	int32_t cc[NP], sc[NP];
-#define SSLM_PAIR(k)                                       \
-	const int p = min((int)threadIdx.x + k * BS, P - 1);     \
-	const bool live = (int)threadIdx.x + k * BS < P;         \
-	const bool isq = p < Q, isk = !isq && p < Q + KP;        \
-	const int kvi = isq ? 0 : p - (isk ? Q : Q + KP); /* K or V pair */
+	// slot k of this thread: its pair p (clamped; live: inside the row), q, K or V, the pair within K or V
+#define SSLM_PAIR(k)                                                                                   \
+	const int i0 = (int)threadIdx.x + (EQ && k >= EQ ? k - EQ : k) * BS;                                 \
+	const int p = EQ ? (k < EQ ? min(i0, Q - 1) : Q + min(i0, KVH - 1)) : min(i0, P - 1);                \
+	const bool live = i0 < (EQ ? (k < EQ ? Q : KVH) : P);                                                \
+	const bool isq = EQ ? k < EQ : p < Q, isk = !isq && p < Q + KP;                                      \
+	const int kvi = isq ? 0 : p - (isk ? Q : Q + KP);
 #pragma unroll
 	for (int k = 0; k < NP; ++k) {
 		SSLM_PAIR(k)
@@ -2135,48 +2138,54 @@ __global__ __launch_bounds__(BS) void k_qkv_post(sslm_launch::QkvPostArgs a) {
 		int64_t b0[NP], b1[NP];
 		const bool any_bias = e.seg[0].bias || e.seg[1].bias || e.seg[2].bias;
 		const int64_t rcp = any_bias ? e.in_recip[t] : 0, ein = any_bias ? e.in_scale[t].e : 0;
-#pragma unroll
-		for (int k = 0; k < NP; ++k) {
-			SSLM_PAIR(k)
-			(void)live;
-			uint32_t s0 = 0, s1 = 0;
-#pragma unroll
-			for (int s2 = 0; s2 < RS; ++s2) {  // clamped plane index: no branch, no extra round trip
-				const int2 x = *(const int2*)(row + (size_t)(RS == 1 ? 0 : min(s2, a.raw.splits - 1)) * plane + 2 * p);
-				s0 += RS == 1 || s2 < a.raw.splits ? (uint32_t)x.x : 0u;  // the true sum fits int32; partials wrap harmlessly
-				s1 += RS == 1 || s2 < a.raw.splits ? (uint32_t)x.y : 0u;
-			}
-			acc[k] = make_int2((int)s0, (int)s1);
-			const int jj = isq ? 2 * p : 2 * kvi;
-			const int32_t* fp = (isq ? e.seg[0].fold : (isk ? e.seg[1].fold : e.seg[2].fold)) + 3 * jj;
-#pragma unroll
-			for (int i = 0; i < 6; ++i) f[k][i] = fp[i];
-			const int64_t* bp = isq ? e.seg[0].bias : (isk ? e.seg[1].bias : e.seg[2].bias);
-			b0[k] = bp ? bp[jj] : 0;
-			b1[k] = bp ? bp[jj + 1] : 0;
-		}
 		bool ok = true;
+		// from five slots on in parts of EQ slots, so that one part's operands are held at a time
+		constexpr int G = EQ && NP >= 5 ? EQ : NP;
 #pragma unroll
-		for (int k = 0; k < NP; ++k) {
-			SSLM_PAIR(k)
-			v0[k] = fold_bounded(acc[k].x, fold_consts(f[k][0], f[k][1], f[k][2]));
-			v1[k] = fold_bounded(acc[k].y, fold_consts(f[k][3], f[k][4], f[k][5]));
-			const int8_t* lb = isq ? e.seg[0].lora_b : (isk ? e.seg[1].lora_b : e.seg[2].lora_b);
-			if (lb) {
-				const int8_t* lu = isq ? e.seg[0].lora_u : (isk ? e.seg[1].lora_u : e.seg[2].lora_u);
-				const int32_t* df = isq ? e.seg[0].lora_dfold : (isk ? e.seg[1].lora_dfold : e.seg[2].lora_dfold);
+		for (int k0 = 0; k0 < NP; k0 += G) {
+#pragma unroll
+			for (int k = k0; k < min(k0 + G, NP); ++k) {
+				SSLM_PAIR(k)
+				(void)live;
+				uint32_t s0 = 0, s1 = 0;
+#pragma unroll
+				for (int s2 = 0; s2 < RS; ++s2) {  // clamped plane index: no branch, no extra round trip
+					const int2 x = *(const int2*)(row + (size_t)(RS == 1 ? 0 : min(s2, a.raw.splits - 1)) * plane + 2 * p);
+					s0 += RS == 1 || s2 < a.raw.splits ? (uint32_t)x.x : 0u;  // the true sum fits int32; partials wrap harmlessly
+					s1 += RS == 1 || s2 < a.raw.splits ? (uint32_t)x.y : 0u;
+				}
+				acc[k] = make_int2((int)s0, (int)s1);
 				const int jj = isq ? 2 * p : 2 * kvi;
-				v0[k] += lora_delta_cold(lb, lu, df, e.rank, t, jj);
-				v1[k] += lora_delta_cold(lb, lu, df, e.rank, t, jj + 1);
+				const int32_t* fp = (isq ? e.seg[0].fold : (isk ? e.seg[1].fold : e.seg[2].fold)) + 3 * jj;
+#pragma unroll
+				for (int i = 0; i < 6; ++i) f[k][i] = fp[i];
+				const int64_t* bp = isq ? e.seg[0].bias : (isk ? e.seg[1].bias : e.seg[2].bias);
+				b0[k] = bp ? bp[jj] : 0;
+				b1[k] = bp ? bp[jj + 1] : 0;
 			}
-			if (isq ? e.seg[0].bias != nullptr : (isk ? e.seg[1].bias != nullptr : e.seg[2].bias != nullptr)) {
-				int64_t t0 = 0, t1 = 0;
-				const bool o = bias_term(b0[k], rcp, ein, v0[k], &t0) & bias_term(b1[k], rcp, ein, v1[k], &t1);
-				v0[k] += t0;
-				v1[k] += t1;
-				if (live && !o) ok = false;
+#pragma unroll
+			for (int k = k0; k < min(k0 + G, NP); ++k) {
+				SSLM_PAIR(k)
+				v0[k] = fold_bounded(acc[k].x, fold_consts(f[k][0], f[k][1], f[k][2]));
+				v1[k] = fold_bounded(acc[k].y, fold_consts(f[k][3], f[k][4], f[k][5]));
+				const int8_t* lb = isq ? e.seg[0].lora_b : (isk ? e.seg[1].lora_b : e.seg[2].lora_b);
+				if (lb) {
+					const int8_t* lu = isq ? e.seg[0].lora_u : (isk ? e.seg[1].lora_u : e.seg[2].lora_u);
+					const int32_t* df = isq ? e.seg[0].lora_dfold : (isk ? e.seg[1].lora_dfold : e.seg[2].lora_dfold);
+					const int jj = isq ? 2 * p : 2 * kvi;
+					v0[k] += lora_delta_cold(lb, lu, df, e.rank, t, jj);
+					v1[k] += lora_delta_cold(lb, lu, df, e.rank, t, jj + 1);
+				}
+				if (isq ? e.seg[0].bias != nullptr : (isk ? e.seg[1].bias != nullptr : e.seg[2].bias != nullptr)) {
+					int64_t t0 = 0, t1 = 0;
+					const bool o = bias_term(b0[k], rcp, ein, v0[k], &t0) & bias_term(b1[k], rcp, ein, v1[k], &t1);
+					v0[k] += t0;
+					v1[k] += t1;
+					if (live && !o) ok = false;
+				}
+				if (live && isq) qmx = max(qmx, max(sat_abs_u32(v0[k]), sat_abs_u32(v1[k])));
 			}
-			if (live && isq) qmx = max(qmx, max(sat_abs_u32(v0[k]), sat_abs_u32(v1[k])));
+			if (G < NP) __builtin_amdgcn_sched_barrier(0);
 		}
 		if (!ok) qmx = kBad32;
 	} else {
@@ -2186,16 +2195,18 @@ __global__ __launch_bounds__(BS) void k_qkv_post(sslm_launch::QkvPostArgs a) {
 		longlong2 kr[NP];
 #pragma unroll
 		for (int k = 0; k < NP; ++k) {
-			const int p = min((int)threadIdx.x + k * BS, P - 1);
+			SSLM_PAIR(k)
+			(void)live, (void)kvi, (void)isk;
 			qr[k] = make_int2(0, 0);
 			kr[k] = make_longlong2(0, 0);
-			if (p < Q) qr[k] = qf[p];
+			if (isq) qr[k] = qf[p];
 			else kr[k] = kv[p - Q];
 		}
-		qmx = part_max32_fixed<BS, (2 * NP + 15) / 16>(a.q_maxpart, 0, H / 16, t);  // H <= 2 NP BS
+		qmx = part_max32_fixed<BS, (2 * (EQ ? EQ : NP) + 15) / 16>(a.q_maxpart, 0, H / 16, t);  // H <= 2 EQ (NP) BS
 #pragma unroll
 		for (int k = 0; k < NP; ++k) {
-			const bool isq = (int)threadIdx.x + k * BS < Q;
+			SSLM_PAIR(k)
+			(void)live, (void)kvi, (void)isk;
 			v0[k] = isq ? (int64_t)qr[k].x : (int64_t)kr[k].x;
 			v1[k] = isq ? (int64_t)qr[k].y : (int64_t)kr[k].y;
 		}
@@ -4825,15 +4836,27 @@ void rmsnorm(const RowNormArgs& a, int M, int H, const TokenInfo* tok, int32_t* 
 
 void qkv_post(const QkvPostArgs& a, hipStream_t s) {
 	const int need = row_ept(a.H / 2 + a.NKV * a.D, kRowBS);
-#define X(E)                                                                                          \
-	if (need <= E) {                                                                                  \
-		if (!a.raw.part) hipLaunchKernelGGL((k_qkv_post<kRowBS, E, 0>), dim3(a.M), dim3(kRowBS), 0, s, a); \
-		else if (a.raw.splits == 1) hipLaunchKernelGGL((k_qkv_post<kRowBS, E, 1>), dim3(a.M), dim3(kRowBS), 0, s, a); \
-		else hipLaunchKernelGGL((k_qkv_post<kRowBS, E, kMaxRawSplits>), dim3(a.M), dim3(kRowBS), 0, s, a); \
-		return;                                                                                       \
+#define SSLM_QKV(E, EQ)                                                                                                \
+	{                                                                                                           \
+		if (!a.raw.part) hipLaunchKernelGGL((k_qkv_post<kRowBS, E, EQ, 0>), dim3(a.M), dim3(kRowBS), 0, s, a);     \
+		else if (a.raw.splits == 1) hipLaunchKernelGGL((k_qkv_post<kRowBS, E, EQ, 1>), dim3(a.M), dim3(kRowBS), 0, s, a); \
+		else hipLaunchKernelGGL((k_qkv_post<kRowBS, E, EQ, kMaxRawSplits>), dim3(a.M), dim3(kRowBS), 0, s, a);     \
+		return;                                                                                                 \
 	}
-	X(1) X(2) X(3) X(5) X(8) X(12)  // at most 8 of q (H / 2 <= 8 kRowBS) and 4 of K and V
+	// up to three slots a thread the even spread (hidden 1536, 16 / 2,048 rows: 4.9 / 17.4 us, against 5.3 / 19.3
+	// with q, K and V in slots of their own and 128-bit landings); from four on its slots of every kind
+	// cost more than they spare: 16 / 128 / 2,048 rows evenly and by kind, hidden 3584 6.9 / 8.3 / 34.1 and
+	// 6.1 / 7.3 / 23.8 us, hidden 4096 with 1,024 K columns 8.6 / 9.9 / 61.1 and 7.0 / 8.3 / 31.3
+#define X(E) \
+	if (need <= E) SSLM_QKV(E, 0)
+	X(1) X(2) X(3)
 #undef X
+	const int nq = row_ept(a.H / 2, kRowBS), nkv = row_ept(a.NKV * a.D, kRowBS);
+#define X(Q, KV) \
+	if (nq <= Q && nkv <= KV) SSLM_QKV(Q + KV, Q)
+	X(2, 2) X(2, 4) X(3, 1) X(3, 2) X(4, 1) X(4, 2) X(4, 4) X(8, 2) X(8, 4)  // H / 2 <= 8 kRowBS, K and V <= 4 kRowBS
+#undef X
+#undef SSLM_QKV
 	no_instance("qkv_post", a.H);
 }
 
