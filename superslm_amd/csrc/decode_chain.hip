@@ -465,6 +465,11 @@ static int act_ntb(int N, int splits) {
 	return 0;
 }
 
+// Rows past kChainRows and the second to fourth row's residual: the header's figures.  The other limits are
+// what the kernels hold, not lines between two measured forms: k_act_gemv writes the split-K planes
+// that the down GEMV has past I = 4096 only (up to there it runs unsplit in k_gemv_pk); a wave reads one maximum per
+// lane (NH); an adapter's u = A x needs the codes in memory before the GEMV that k_funnel_gemv and
+// k_act_gemv derive them in, so the caller takes no layer with an adapter here.
 bool decode_chain_ok(int M, int H, int NH, int KVH, int I) {
 	if (M < 1 || M > kChainRows || H % 128 || I % 128 || I <= 4096 || NH > 64) return false;
 	const int C = H / 128, cpw = chain_cpw(C), ac = act_cpw(I / 128), planes = packed_planes(M, H, I);

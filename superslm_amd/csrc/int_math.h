@@ -11,8 +11,8 @@
 #include <stdint.h>
 
 #define SSLM_HD __host__ __device__ __forceinline__
-// Rarely taken slow paths stay out of line: a kernel's latency-bound row code runs once per
-// launch from a cold instruction cache, so its size costs more than a call on the rare path.
+// Rarely taken slow paths stay out of line: inlined 128-bit forms take registers from, and put
+// instructions into, latency-bound row code that almost never needs them.
 #define SSLM_COLD __host__ __device__ inline __attribute__((noinline))
 
 namespace sslm {
@@ -289,7 +289,7 @@ struct FunnelOut {
 // (relative error near 2^-50), rounded to an integer y: at most 1/2 + 2^-17 from the quotient, which lies
 // in (2^31, 2^32].  2^62 - y dn is then below 2^31 in magnitude, so one fma gives it exactly, and one
 // step of the reference's correction rule finishes it, in full-rate double operations (two
-// steps on 64-bit products were 66 instructions of a plan that runs cold, three plans a row).
+// steps on 64-bit products were 66 dependent instructions of a plan, three plans a row).
 // Checked equal to reciprocal_div for every dn in [2^30, 2^31) by tests/reciprocal_norm_check.
 SSLM_HD double reciprocal_norm_d(double dd) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -423,7 +423,7 @@ SSLM_HD int64_t clamp_code(int64_t v) { return v > 127 ? 127 : (v < -127 ? -127 
 // x = |branch| f is within 200 * 2^-50 of the exact magnitude below 200, and rounding it half up is exact
 // unless x + 1/2 lies within 1e-9 of an integer.  That band, a product past 2^126 or a quotient past
 // 2^62 (where the 128-bit form wraps) take the exact form out of line: inlined at each value
-// it was most of its kernels' instruction bytes, which a launch fetches cold.
+// it was most of its kernels' code.
 struct LandingScale {
 	double p, f;
 };

@@ -3249,7 +3249,7 @@ __global__ __launch_bounds__(BS) void k_attention(sslm_launch::AttnArgs a) {
 // tokens and their decoding 293.6 -> 280.4 ms).  4-wave blocks, held to 3 a CU, have no registers
 // for either (2,048-token 7B attention 321 -> 369 us with them): k_kv_commit runs before them.
 // The general i-exp and quotient of rows past the 32-bit forms are called out of line: inlined eight
-// times they were 10 KB of the kernel, fetched cold by each launch (4-12 tokens 12.7 -> 11.8 us).
+// times they were 10 KB of the kernel (4-12 tokens 12.7 -> 11.8 us without).
 // A short tile is one chain of dependent phases, so nothing waits that need not: the last wave derives
 // the i-exp constants (4,000 cycles of 25,000) while the others run pass 1, the committed rows are
 // loaded at entry with the operands (the round trip was 3,200), rows reduce by DPP rotations instead of
@@ -4761,7 +4761,11 @@ PrefillPlan prefill_plan(int M, int N, int K, bool split_ok) {
 	p.splits = 1;
 	// narrow: raw output of 64 x 64 tiles, one plane, for consumers that add raw planes.  Every
 	// small tile streams its whole K of both operands, so long K (the down projection) keeps
-	// the large tiles with K split into planes.
+	// the large tiles with K split into planes.  Raw launches, us in 64 x 64 tiles / 128- or 256-row tiles with
+	// K split / the same unsplit: N = K = 1536 at 512, 1,024, 2,048 rows 6.1 / 10.4 / 12.8, 8.0 / 11.6 / 13.2,
+	// 12.0 / 23.5 / 14.2; N = 4608, K = 3584 at 256, 512 rows 12.6 / 13.5 / 19.6, 20.2 / 27.5 / 20.4.  The
+	// line is too high for deep launches of many rows: N = K = 3584 at 768 rows 20.2 / 28.1 / 20.7, but at
+	// 1,024 24.6 / 29.5 / 21.1 and at 2,048 56.4 / 38.6 / 30.6.
 	p.narrow = split_ok && tiles < kPrefillTargetBlocks && K <= kNarrowMaxK;
 	if (p.narrow) {
 		p.kspan = K;
